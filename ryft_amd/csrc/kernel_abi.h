@@ -255,6 +255,13 @@ struct AttnArgs {
   float scale;
   // element strides of Q, K, V, O in (b, h, s, d) order
   int64_t qs[4], ks[4], vs[4], os[4];
+  // few queries against many keys: the keys of a (batch, head) run in `splits` ranges whose partial results
+  // (unnormalised output, maximum and sum per query: B·H × splits × Sq × (D + 2) floats) go to ws; the range that
+  // arrives last at its (batch, head)'s counter (zero between launches) merges them. splits <= 1: neither is used.
+  int32_t splits;
+  int32_t pad_;
+  float* ws;
+  int32_t* counters;
 };
 
 // ------------------------------------------------------------------------------------------------ dynamic windows

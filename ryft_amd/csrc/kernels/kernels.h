@@ -36,5 +36,10 @@ bool attention_supported(int head_dim);
 // Why the fused attention kernel cannot run these arguments (null: it can). The planner calls it with the operands'
 // byte offsets from their (256-byte aligned) slots in place of pointers, and fuses only when it returns null.
 const char* attention_unsupported(const AttnArgs& a);
+// Name of the kernel launch_attention() picks for these arguments (used for profiling labels).
+const char* attention_kernel_name(const AttnArgs& a);
+// Number of key ranges launch_attention runs these arguments in when given a workspace of
+// B·H × ranges × Sq × (D + 2) floats and B·H zeroed counters (1: it needs neither).
+int attention_plan_splits(const AttnArgs& a);
 
 }  // namespace ryft

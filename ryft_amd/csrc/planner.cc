@@ -2245,9 +2245,19 @@ bool Planner::try_attention(int d2, int target, DType out_dtype, int root) {
   // the launcher's preconditions, checked here on the operands' offsets (slots are 256-byte aligned) so that a
   // graph the kernel cannot run takes the unfused path instead of failing at execute time
   if (attention_unsupported(A)) return false;
+  st.name = attention_kernel_name(A);
   int out = temp_or(target, rn.type);
   st.patches = {{offsetof(AttnArgs, q), vq.slot}, {offsetof(AttnArgs, k), vk.slot}, {offsetof(AttnArgs, v), vv.slot},
                 {offsetof(AttnArgs, o), out}};
+  A.splits = attention_plan_splits(A);
+  if (A.splits > 1) {
+    const int ws = new_slot(Slot::TEMP, TensorType{DType::F32, {B * H, A.splits, Sq, Dh + 2}});
+    st.patches.push_back({offsetof(AttnArgs, ws), ws});
+    const TensorType ct{DType::S32, {B * H}};
+    const int cs = new_slot(Slot::CONSTANT, ct);
+    plan_.slots[cs].literal.assign((size_t)ct.bytes(), 0);
+    st.patches.push_back({offsetof(AttnArgs, counters), cs});
+  }
   double pairs = causal ? (double)Sq * (double)(Sk + 1) / 2.0 : (double)Sq * (double)Sk;  // Sq == Sk for causal
   st.flops = 4.0 * (double)B * (double)H * (double)Dh * pairs;
   st.bytes = (double)(Qt.bytes() + Kt.bytes() + Vt.bytes() + rn.type.bytes());
