@@ -481,7 +481,9 @@ __device__ __forceinline__ uint32_t out_bits(uint32_t x, bool is_float) {
 // cache write-back or invalidation is needed between the ranges and the one that finishes the tile. The loads are
 // not seen by the compiler's wait-count tracking: wait_loads() completes them.
 __device__ __forceinline__ void store_coherent16(void* p, const u32x4& v) {
-  asm volatile("global_store_dwordx4 %0, %1, off sc1" ::"v"(p), "v"(v) : "memory");
+  // (the two wait states a store of more than 8 bytes needs before its data registers are written again: the compiler
+  // sees no store in an asm statement and adds none, and a vector instruction right behind it changed the stored words)
+  asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
 }
 __device__ __forceinline__ u32x4 load_coherent16(const void* p) {
   u32x4 r;
