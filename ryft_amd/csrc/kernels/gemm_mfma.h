@@ -3,15 +3,21 @@
 // GEMM kernels for gfx950 (see also k_gemm_dispatch.hip).
 //
 // MFMA path: one workgroup computes a BM×BN tile of C[b] = A[b]·B[b]ᵀ (B addressed as [n, k]); WM×WN wavefronts
-// each own a (BM/WM)×(BN/WN) sub-tile made of 32×32 MFMA tiles. Full tiles of a K-contiguous A go from global memory
-// straight into LDS (buffer_load ... lds) in unpadded, XOR-swizzled K-packed rows (each row holds BK consecutive k of
-// one m), together with B — K-packed the same way, or, when its contiguous dimension is n (row-major [K, N] weights),
-// as unchanged [k][n] rows read back with transposing LDS reads — in two or three LDS stages, so no register staging
-// and no LDS store instructions are needed. Edge tiles and m-contiguous A operands take a register-staged path
-// instead: buffer loads one k-tile ahead into registers, padded LDS rows, m / n-contiguous operands transposed in
+// each own a (BM/WM)×(BN/WN) sub-tile made of 32×32 MFMA tiles. 16- and 8-bit operands go from global memory straight
+// into LDS (buffer_load ... lds) in unpadded, XOR-swizzled rows — K-packed (each row holds BK consecutive k of one m or
+// n), or, for an operand contiguous along its free dimension, unchanged [k][m] / [k][n] rows read back with transposing
+// LDS reads — in two to four LDS stages, so no register staging and no LDS store instructions are needed, and no
+// transpose pass over HBM exists. f32 operands, and a K-contiguous f8 B that is widened to bf16, take a register-staged
+// path instead: buffer loads one k-tile ahead into registers, padded LDS rows, m / n-contiguous operands transposed in
 // registers with v_perm_b32 on their way into LDS. Either way LDS fragments are double-buffered in registers across
-// k-steps and across the one barrier per k-tile, and no separate transpose pass over HBM is needed. Workgroups are
-// mapped onto the 8 XCDs so that the tiles one XCD computes share A row-panels and B column-panels in that XCD's L2.
+// k-steps and across the one barrier per k-tile. Workgroups are mapped onto the 8 XCDs so that the tiles one XCD computes
+// share A row-panels and B column-panels in that XCD's L2.
+//
+// Measured (kernel times, before: register-staged edge tiles of 128×128 only, loads issued behind a branch):
+// 1000³ bf16 17.3 → 8.4 µs (64×64 tiles), Xᵀ·dY of [2048, 4096]ᵀ·[2048, 4096] 103 → 59 µs (256×256, both operands by
+// transposing reads), 16 rows × f8 weights [4096, 14336] twice 77 → 30 µs and [14336, 4096] 172 → 18 µs (32×128 tiles
+// over K ranges). What bounds them: the small tiles the L2-to-LDS rate (about 60 GB/s per CU), the large ones the MFMA
+// issue at the clock the chip holds.
 //
 // Instruction per compute type (all dense, f32 or i32 accumulation):
 //   bf16  v_mfma_f32_32x32x16_bf16      f16  v_mfma_f32_32x32x16_f16
@@ -340,12 +346,14 @@ __device__ __forceinline__ uint2 lds_read_tr8(const char* p) {
 // need 8 distinct positions. Period 16 rows.
 __device__ __forceinline__ int swz_k128(int r) { return (r >> 1) & 7; }
 // [k][n] rows read with transposing reads (32 lanes per pass): 16-bit rows (≥ 256 bytes): 4 consecutive rows × 4
-// consecutive chunks, so the 4 rows' chunk quads go to distinct quads (period 4); 8-bit rows of ≥ 256 bytes: 8 rows
+// consecutive chunks, so the 4 rows' chunk quads go to distinct quads (period 4; rows of 128 bytes: the even and the
+// odd rows fall in different bank halves, two quads each); 8-bit rows of ≥ 256 bytes: 8 rows
 // × 2 chunks (period 8); 8-bit rows of 128 bytes: the even and the odd rows of 8 fall in different bank halves, 4 rows
 // × 2 chunks each (period 8).
 template <int ES, int RB>
 __device__ __forceinline__ int swz_tr(int r) {
-  if constexpr (ES == 2) return 4 * (r & 3);
+  if constexpr (ES == 2 && RB == 128) return 4 * ((r >> 1) & 1);
+  else if constexpr (ES == 2) return 4 * (r & 3);
   else if constexpr (RB >= 256) return 2 * (r & 7);
   else return 2 * ((r >> 1) & 3);
 }
@@ -393,6 +401,11 @@ __device__ __forceinline__ void dma_barrier() {
   asm volatile("s_waitcnt vmcnt(%[n]) lgkmcnt(0)\n\ts_barrier" ::[n] "n"(N) : "memory");
 }
 
+// Joins the workgroup barrier once this wave's LDS stores are done, leaving its DMA loads in flight.
+__device__ __forceinline__ void dma_barrier_keep() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
 template <int KIND, int BM, int BN, int BK, int WM, int WN, bool A_R, bool B_R, bool DUAL, bool EDGE = false>
 struct MfmaCfg {
   using M = Mma<KIND>;
@@ -412,20 +425,27 @@ struct MfmaCfg {
   static constexpr int BLES = BTR ? BES : ESIZE;
   static constexpr int LDB = BN * BLES + (BLES == 2 ? 64 : 32);
   static constexpr int BREG = BTR ? BK * LDB : BN * LDK;  // bytes of one B operand tile
-  // DMA: full tiles of a K-contiguous A and a B that reaches LDS unchanged (n-contiguous 16- / 8-bit, or K-contiguous
-  // without widening) go from global memory straight into LDS (buffer_load ... lds, 16 bytes per lane): unpadded rows
-  // whose 16-byte chunks are XOR-swizzled per row (so that the fragment reads stay conflict-free), no register
-  // staging and no LDS stores; NST stages (three when they fit) keep the loads two k-tiles ahead.
-  static constexpr int RBA = BK * ESIZE;                       // bytes per A row (and per K-contiguous B row)
-  static constexpr int RBB = BTR ? BN * BLES : BK * ESIZE;     // bytes per B row ([k][n] rows when BTR)
-  static constexpr bool DMA = !EDGE && !A_R && ESIZE <= 2 && (BTR || BES == ESIZE) && RBA == 128 &&
-                              (BM * RBA) % (1024 * WM * WN) == 0 && (BTR ? BK : BN) * RBB % (1024 * WM * WN) == 0 &&
-                              (!BTR || RBB == 128 || RBB == 256 || RBB == 512);
-  static constexpr int BREG_D = BTR ? BK * RBB : BN * RBA;
-  static constexpr int STAGE_D = BM * RBA + NB * BREG_D;
-  // three stages when they fit the 160 KB of LDS and two stages would already leave room for one workgroup only
-  static constexpr int NST = DMA && 3 * STAGE_D <= 163840 && 2 * STAGE_D > 163840 / 2 ? 3 : 2;
+  // DMA: operands that reach LDS unchanged (16- and 8-bit types; not a K-contiguous f8 B that is widened on its way) go
+  // from global memory straight into LDS (buffer_load ... lds, 16 bytes per lane): unpadded rows whose 16-byte chunks
+  // are XOR-swizzled per row (so that the fragment reads stay conflict-free), no register staging and no LDS stores.
+  // ATR: an m-contiguous A is kept as [k][m] rows, like an n-contiguous B, and read with the transposing LDS reads.
+  static constexpr int NW = WM * WN;
+  static constexpr bool ATR = A_R && ESIZE <= 2;
+  static constexpr int AROWS = ATR ? BK : BM, RBA = ATR ? BM * ESIZE : BK * ESIZE;      // LDS rows of A, bytes per row
+  static constexpr int BROWS = BTR ? BK : BN, RBB = BTR ? BN * BLES : BK * ESIZE;       // the same of B
+  static constexpr bool tr_row(int rb) { return rb == 128 || rb == 256 || rb == 512; }
+  static constexpr bool DMA = ESIZE <= 2 && (BTR || BES == ESIZE) && BK * ESIZE == 128 &&
+                              (AROWS * RBA) % (1024 * NW) == 0 && (BROWS * RBB) % (1024 * NW) == 0 &&
+                              (!ATR || tr_row(RBA)) && (!BTR || tr_row(RBB));
+  static constexpr int AREG_D = AROWS * RBA, BREG_D = BROWS * RBB;
+  static constexpr int STAGE_D = AREG_D + NB * BREG_D;
+  // Stages: four for the small tiles, whose k-tiles multiply for less time than a load takes to arrive; three where
+  // they fit the 160 KB of LDS and two would already leave room for one workgroup only; else two.
+  static constexpr bool SMALL = BM * BN <= 64 * 128;
+  static constexpr int NST = DMA && SMALL ? 4 : DMA && 3 * STAGE_D <= 163840 && 2 * STAGE_D > 163840 / 2 ? 3 : 2;
   static constexpr int STAGE = DMA ? STAGE_D : BM * LDK + NB * BREG;
+  // split-K is compiled in for every tile that a plan splits: all but the 256-row ones
+  static constexpr bool SPLIT = BM * BN * NB <= 128 * 256;
   static_assert(BK % MK == 0, "BK must be a multiple of the MFMA K");
   static_assert(WTM % 32 == 0 && WTN % 32 == 0, "wave tile must be a multiple of 32");
   // epilogue rounds: the largest number of 32-row tile-rows (dividing TM) whose f32 patches fit in the LDS the two
@@ -676,10 +696,12 @@ __device__ __forceinline__ void splitk_epilogue_oct(const GemmArgs& G, int64_t e
 
 // The K range that finishes a BM×BN tile last: sums the S ranges' partial sums in range order (the reduction
 // kernel's order) and applies the epilogue, eight consecutive elements per thread and step, with the loads of
-// 16 / S steps in flight together.
-template <bool INT, int S, int BM, int BN, int THREADS>
+// 16 / S steps in flight together. EDGE (N a multiple of 8): steps past the tile's last row end the loop, positions past
+// M or N are read as the last valid ones and not stored.
+template <bool INT, bool DUAL, bool EDGE, int S, int BM, int BN, int THREADS>
 __device__ __forceinline__ void splitk_finish_tile(const GemmArgs& G, int b, int m0, int n0, int tid) {
-  constexpr int OCTS = BM * BN / 8, PER = OCTS / THREADS, B0 = S >= 16 ? 1 : 16 / S, BATCH = PER < B0 ? PER : B0;
+  constexpr int NB = DUAL ? 2 : 1;
+  constexpr int OCTS = BM * BN / 8, PER = OCTS / THREADS, B0 = S * NB >= 16 ? 1 : 16 / (S * NB), BATCH = PER < B0 ? PER : B0;
   static_assert(OCTS % THREADS == 0 && PER % BATCH == 0, "finish layout");
   const int64_t slice = (int64_t)G.batch * G.M * G.N;
   const uint32_t* ws = (const uint32_t*)G.ws;
@@ -687,43 +709,57 @@ __device__ __forceinline__ void splitk_finish_tile(const GemmArgs& G, int b, int
     return INT ? (uint32_t)((int32_t)a + (int32_t)x) : __float_as_uint(__uint_as_float(a) + __uint_as_float(x));
   };
   for (int o0 = 0; o0 < PER; o0 += BATCH) {
-    u32x4 w[BATCH][S][2];
+    if (EDGE && m0 + o0 * THREADS / (BN / 8) >= G.M) break;
+    u32x4 w[BATCH][S][NB][2];
     int64_t e0[BATCH];
 #pragma unroll
     for (int q = 0; q < BATCH; ++q) {
       const int oc = tid + (o0 + q) * THREADS;
-      const int r = oc / (BN / 8), c = (oc % (BN / 8)) * 8;
-      e0[q] = ((int64_t)b * G.M + m0 + r) * G.N + n0 + c;
+      int r = m0 + oc / (BN / 8), c = n0 + (oc % (BN / 8)) * 8;
+      if constexpr (EDGE) r = min(r, G.M - 1), c = min(c, G.N - 8);
+      e0[q] = ((int64_t)b * G.M + r) * G.N + c;
 #pragma unroll
-      for (int s = 0; s < S; ++s) {
-        w[q][s][0] = load_coherent16(ws + s * slice + e0[q]);
-        w[q][s][1] = load_coherent16(ws + s * slice + e0[q] + 4);
-      }
+      for (int s = 0; s < S; ++s)
+#pragma unroll
+        for (int k = 0; k < NB; ++k) {
+          const uint32_t* p = ws + (s * NB + k) * slice + e0[q];
+          w[q][s][k][0] = load_coherent16(p);
+          w[q][s][k][1] = load_coherent16(p + 4);
+        }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 #pragma unroll
     for (int q = 0; q < BATCH; ++q)
 #pragma unroll
-      for (int s = 0; s < S; ++s) {
-        asm volatile("" : "+v"(w[q][s][0]));
-        asm volatile("" : "+v"(w[q][s][1]));
-      }
+      for (int s = 0; s < S; ++s)
+#pragma unroll
+        for (int k = 0; k < NB; ++k) {
+          asm volatile("" : "+v"(w[q][s][k][0]));
+          asm volatile("" : "+v"(w[q][s][k][1]));
+        }
 #pragma unroll
     for (int q = 0; q < BATCH; ++q) {
-      uint32_t v[8];
+      uint32_t v[NB][8];
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        v[4 * h] = w[q][0][h].x, v[4 * h + 1] = w[q][0][h].y, v[4 * h + 2] = w[q][0][h].z, v[4 * h + 3] = w[q][0][h].w;
-      }
-#pragma unroll
-      for (int s = 1; s < S; ++s)
+      for (int k = 0; k < NB; ++k) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-          v[4 * h] = add(v[4 * h], w[q][s][h].x), v[4 * h + 1] = add(v[4 * h + 1], w[q][s][h].y);
-          v[4 * h + 2] = add(v[4 * h + 2], w[q][s][h].z), v[4 * h + 3] = add(v[4 * h + 3], w[q][s][h].w);
+          const u32x4 x = w[q][0][k][h];
+          v[k][4 * h] = x.x, v[k][4 * h + 1] = x.y, v[k][4 * h + 2] = x.z, v[k][4 * h + 3] = x.w;
         }
+#pragma unroll
+        for (int s = 1; s < S; ++s)
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const u32x4 x = w[q][s][k][h];
+            v[k][4 * h] = add(v[k][4 * h], x.x), v[k][4 * h + 1] = add(v[k][4 * h + 1], x.y);
+            v[k][4 * h + 2] = add(v[k][4 * h + 2], x.z), v[k][4 * h + 3] = add(v[k][4 * h + 3], x.w);
+          }
+      }
       const int oc = tid + (o0 + q) * THREADS;
-      splitk_epilogue_oct<INT, false>(G, e0[q], b, m0 + oc / (BN / 8), n0 + (oc % (BN / 8)) * 8, v, v);
+      const int r = m0 + oc / (BN / 8), c = n0 + (oc % (BN / 8)) * 8;
+      if (EDGE && (r >= G.M || c >= G.N)) continue;
+      splitk_epilogue_oct<INT, DUAL>(G, e0[q], b, r, c, v[0], v[NB - 1]);
     }
   }
 }
@@ -778,8 +814,9 @@ __device__ __forceinline__ void epi_round(const GemmArgs& G, int b, int m0, int 
   else epi_round_mr<INT, DUAL, false, WTN, PITCH, ROWS, EDGE>(G, b, m0, n0, reg, reg2, lane);
 }
 
-// EDGE: any M, N (partial tiles at the edges: bounded loads, masked stores) and any K that is a multiple of the
-// 16-byte vector (the last k-tile loads zeros past K); no split-K.
+// EDGE: any M, N (partial tiles at the edges: bounded or clamped loads, masked stores) and any K that is a multiple of
+// the 16-byte vector of each K-contiguous operand (the last k-tile multiplies zeros past K); split-K with N a multiple
+// of 8.
 template <int KIND, int BM, int BN, int BK, int WM, int WN, bool A_R, bool B_R, bool DUAL, bool EDGE>
 __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const GemmArgs G) {
   using C = MfmaCfg<KIND, BM, BN, BK, WM, WN, A_R, B_R, DUAL, EDGE>;
@@ -840,36 +877,67 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const GemmArgs 
       if constexpr (DUAL) acc2[i][j] = Acc{};
     }
 
-  // k-tiles of this workgroup's K range
-  const int KT = EDGE ? (G.K + BK - 1) / BK : (G.splits > 1 ? G.K / BK / G.splits : G.K / BK);
-  const int kt0 = split * KT;
+  // k-tiles of this workgroup's K range (the last range of an edge kernel may be shorter; none is empty)
+  const int KTA = EDGE ? (G.K + BK - 1) / BK : G.K / BK;
+  const int KTR = nsplit > 1 ? (KTA + nsplit - 1) / nsplit : KTA;
+  const int kt0 = split * KTR;
+  const int KT = EDGE ? min(KTR, KTA - kt0) : KTR;
   if constexpr (C::DMA) {
     // ---- operand tiles straight from global memory into LDS (buffer_load ... lds), NST stages
-    constexpr int NW = WM * WN, NST = C::NST, RBA = C::RBA, RBB = C::RBB;
-    constexpr int UA = RBA / 16, R1A = 1024 / RBA, PA = BM * RBA / 1024 / NW;  // chunks / row, rows / piece, pieces
-    constexpr int BROWS = C::BTR ? BK : BN;
-    constexpr int UB = RBB / 16, R1B = 1024 / RBB, PB = BROWS * RBB / 1024 / NW;
+    constexpr int NW = C::NW, NST = C::NST, RBA = C::RBA, RBB = C::RBB;
+    constexpr int UA = RBA / 16, R1A = 1024 / RBA, PA = C::AREG_D / 1024 / NW;  // chunks / row, rows / piece, pieces
+    constexpr int UB = RBB / 16, R1B = 1024 / RBB, PB = C::BREG_D / 1024 / NW;
     constexpr int OPS = PA + C::NB * PB;  // DMA loads per wave per k-tile
-    constexpr int BREG = C::BREG_D;
-    static_assert((NW * R1A) % 16 == 0 && (NW * R1B) % (C::BTR ? 8 : 16) == 0, "piece rows must keep the swizzle");
-    static_assert(OPS <= 63, "vmcnt range");
+    constexpr int AREG = C::AREG_D, BREG = C::BREG_D;
+    static_assert((NW * R1A) % (C::ATR ? 8 : 16) == 0 && (NW * R1B) % (C::BTR ? 8 : 16) == 0,
+                  "piece rows must keep the swizzle");
+    static_assert((NST - 1) * OPS <= 63, "vmcnt range");
     const int wave_u = __builtin_amdgcn_readfirstlane(wave);
-    // per-lane source offsets of piece 0 (pieces i of a wave are i·NW·R1 rows further: a scalar offset)
-    const int64_t a_rs = G.A.sr * ES;
-    const int ra = wave_u * R1A + lane / UA;
-    const int a_voff = (int)(ra * a_rs) + 16 * ((lane % UA) ^ swz_k128(ra));
-    const int a_pstep = (int)(NW * R1A * a_rs);
+    // per-lane source: row r0 (+ i·NW·R1 for piece i) and 16-byte chunk c (the same for every piece: the swizzle's
+    // period divides NW·R1)
+    auto asw = [&](int r) { if constexpr (C::ATR) return swz_tr<ES, RBA>(r); else return swz_k128(r); };
     auto bsw = [&](int r) { if constexpr (C::BTR) return swz_tr<C::BLES, RBB>(r); else return swz_k128(r); };
-    const int rb = wave_u * R1B + lane / UB;
-    const int64_t b_rs = C::BTR ? G.B.sk * BES : G.B.sr * ES;
-    const int b_voff = (int)(rb * b_rs) + 16 * ((lane % UB) ^ bsw(rb));
-    const int b_pstep = (int)(NW * R1B * b_rs);
-    int b2_voff = 0, b2_pstep = 0;
-    if constexpr (DUAL) {
-      const int64_t b2_rs = C::BTR ? G.B2.sk * BES : G.B2.sr * ES;
-      b2_voff = (int)(rb * b2_rs) + 16 * ((lane % UB) ^ bsw(rb));
-      b2_pstep = (int)(NW * R1B * b2_rs);
-    }
+    const int64_t a_rs = (C::ATR ? G.A.sk : G.A.sr) * ES;
+    const int ra = wave_u * R1A + lane / UA, ca = (lane % UA) ^ asw(ra);
+    const int64_t b_rs = (C::BTR ? G.B.sk : G.B.sr) * BES;
+    const int rb = wave_u * R1B + lane / UB, cb = (lane % UB) ^ bsw(rb);
+    const int64_t b2_rs = DUAL ? (C::BTR ? G.B2.sk : G.B2.sr) * BES : 0;
+    // Edge tiles: rows and chunks past M, N or K are read as the last valid ones (every access stays inside the
+    // operand, whose rows are whole vectors). Rows of C past M or N are not stored, and the k positions past K are
+    // zeroed in LDS (zero_tail) once their tile has arrived. kv: the k positions of the tile that exist.
+    constexpr int VA = 16 / ES, VB = 16 / BES;
+    const int mv = EDGE ? G.M - m0 : 0, nv = EDGE ? G.N - n0 : 0;
+    auto off_a = [&](int i, int kv) {
+      const int r = ra + i * NW * R1A;
+      return C::ATR ? min(r, kv - 1) * (int)a_rs + 16 * min(ca, (mv + VA - 1) / VA - 1)
+                    : min(r, mv - 1) * (int)a_rs + 16 * min(ca, (kv + VA - 1) / VA - 1);
+    };
+    auto off_b = [&](int i, int kv, int64_t rs) {
+      const int r = rb + i * NW * R1B;
+      return C::BTR ? min(r, kv - 1) * (int)rs + 16 * min(cb, (nv + VB - 1) / VB - 1)
+                    : min(r, nv - 1) * (int)rs + 16 * min(cb, (kv + VB - 1) / VB - 1);
+    };
+    const int ktail = EDGE ? G.K - (KTA - 1) * BK : BK;  // k positions of the last k-tile
+    int a_off[EDGE ? PA : 1], b_off[EDGE ? PB : 1], b2_off[EDGE && DUAL ? PB : 1];
+    auto set_offsets = [&](int kv) {
+      if constexpr (EDGE) {
+#pragma unroll
+        for (int i = 0; i < PA; ++i) a_off[i] = off_a(i, kv);
+#pragma unroll
+        for (int i = 0; i < PB; ++i) {
+          b_off[i] = off_b(i, kv, b_rs);
+          if constexpr (DUAL) b2_off[i] = off_b(i, kv, b2_rs);
+        }
+      }
+    };
+    set_offsets(BK);
+    // before the loads of k-tile t: the offsets of the last, partial k-tile (nothing is loaded after it)
+    auto before_dma = [&](int t) {
+      if (EDGE && ktail < BK && kt0 + t == KTA - 1) set_offsets(ktail);
+    };
+    const int a_voff = (int)(ra * a_rs) + 16 * ca, a_pstep = (int)(NW * R1A * a_rs);
+    const int b_voff = (int)(rb * b_rs) + 16 * cb, b_pstep = (int)(NW * R1B * b_rs);
+    const int b2_voff = (int)(rb * b2_rs) + 16 * cb, b2_pstep = (int)(NW * R1B * b2_rs);
     auto dma = [&](int t, int st) {
       const int64_t ko = (int64_t)(kt0 + t) * BK;
       char* sb = smem + st * C::STAGE;
@@ -877,29 +945,74 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const GemmArgs 
           __builtin_amdgcn_make_buffer_rsrc((void*)(Ab + ko * G.A.sk * ES), (short)0, -1, 0x00020000);
       const __amdgpu_buffer_rsrc_t rsb =
           __builtin_amdgcn_make_buffer_rsrc((void*)(Bb + ko * G.B.sk * BES), (short)0, -1, 0x00020000);
+      const __amdgpu_buffer_rsrc_t rsb2 =
+          DUAL ? __builtin_amdgcn_make_buffer_rsrc((void*)(B2b + ko * G.B2.sk * BES), (short)0, -1, 0x00020000) : rsb;
+      auto piece = [&](int i) { return sb + (wave_u + i * NW) * 1024; };
 #pragma unroll
-      for (int i = 0; i < PA; ++i) lds_dma16(rsa, sb + (wave_u + i * NW) * 1024, a_voff, i * a_pstep);
-#pragma unroll
-      for (int i = 0; i < PB; ++i) lds_dma16(rsb, sb + BM * RBA + (wave_u + i * NW) * 1024, b_voff, i * b_pstep);
-      if constexpr (DUAL) {
-        const __amdgpu_buffer_rsrc_t rsb2 =
-            __builtin_amdgcn_make_buffer_rsrc((void*)(B2b + ko * G.B2.sk * BES), (short)0, -1, 0x00020000);
-#pragma unroll
-        for (int i = 0; i < PB; ++i)
-          lds_dma16(rsb2, sb + BM * RBA + BREG + (wave_u + i * NW) * 1024, b2_voff, i * b2_pstep);
+      for (int i = 0; i < PA; ++i) {
+        if constexpr (EDGE) lds_dma16(rsa, piece(i), a_off[i], 0);
+        else lds_dma16(rsa, piece(i), a_voff, i * a_pstep);
       }
+#pragma unroll
+      for (int i = 0; i < PB; ++i) {
+        if constexpr (EDGE) lds_dma16(rsb, piece(i) + AREG, b_off[i], 0);
+        else lds_dma16(rsb, piece(i) + AREG, b_voff, i * b_pstep);
+      }
+      if constexpr (DUAL) {
+#pragma unroll
+        for (int i = 0; i < PB; ++i) {
+          if constexpr (EDGE) lds_dma16(rsb2, piece(i) + AREG + BREG, b2_off[i], 0);
+          else lds_dma16(rsb2, piece(i) + AREG + BREG, b2_voff, i * b2_pstep);
+        }
+      }
+    };
+    // Stage st holds the last, partial k-tile, complete in every wave: its k positions from ktail on become zeros (in
+    // both operands: what was read in their place may be an infinity or a NaN), joined by a barrier of its own.
+    auto zero_tail = [&](int st) {
+      char* sb = smem + st * C::STAGE;
+      auto zero_rows = [&](char* base, int rb_, int bytes) {  // [k][...] rows from ktail on
+        for (int o = ktail * rb_ + tid * 16; o < bytes; o += C::THREADS * 16) *(u32x4*)(base + o) = u32x4{0, 0, 0, 0};
+      };
+      auto zero_chunks = [&](char* base, int rows, int v) {  // K-packed rows of 8 chunks
+        for (int o = tid; o < rows * 8; o += C::THREADS)
+          if ((o & 7) >= ktail / v) *(u32x4*)(base + (o >> 3) * 128 + 16 * ((o & 7) ^ swz_k128(o >> 3))) = u32x4{0, 0, 0, 0};
+      };
+      if constexpr (C::ATR) zero_rows(sb, RBA, AREG);
+      else zero_chunks(sb, BM, VA);
+      static_for<0, C::NB>([&](auto bc) {
+        char* base = sb + AREG + decltype(bc)::value * BREG;
+        if constexpr (C::BTR) zero_rows(base, RBB, BREG);
+        else zero_chunks(base, BN, VB);
+      });
+      dma_barrier_keep();
     };
 
     // ---- fragment read addresses (bytes from the stage base)
     constexpr int S = BK / C::MK;
     constexpr int CPL = C::KPACK * ES / 16;  // 16-byte chunks per lane per K-packed fragment (2 for fp8)
     const int half = lane >> 5, l32 = lane & 31;
-    int a_rd[S][CPL];
+    constexpr int NAR = C::ATR ? C::TM : S * CPL;
+    int a_rd[NAR];
+    if constexpr (C::ATR) {
 #pragma unroll
-    for (int s = 0; s < S; ++s)
+      for (int i = 0; i < C::TM; ++i) {
+        if constexpr (ES == 2) {
+          const int kr = 8 * half + ((lane & 15) >> 2);
+          const int ch = (wm * C::WTM + 32 * i) / 8 + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1);
+          a_rd[i] = kr * RBA + 16 * (ch ^ swz_tr<2, RBA>(kr)) + 8 * (lane & 1);
+        } else {
+          const int kr = C::KPACK * half + ((lane & 15) >> 1);
+          const int ch = (wm * C::WTM + 32 * i) / 16 + ((lane >> 4) & 1);
+          a_rd[i] = kr * RBA + 16 * (ch ^ swz_tr<1, RBA>(kr)) + 8 * (lane & 1);
+        }
+      }
+    } else {
 #pragma unroll
-      for (int q = 0; q < CPL; ++q)
-        a_rd[s][q] = (wm * C::WTM + l32) * RBA + 16 * ((s * 2 * CPL + half * CPL + q) ^ swz_k128(l32));
+      for (int s = 0; s < S; ++s)
+#pragma unroll
+        for (int q = 0; q < CPL; ++q)
+          a_rd[s * CPL + q] = (wm * C::WTM + l32) * RBA + 16 * ((s * 2 * CPL + half * CPL + q) ^ swz_k128(l32));
+    }
     constexpr int NBR = C::BTR ? C::TN : S * CPL;
     int b_rd[NBR];
     if constexpr (C::BTR) {
@@ -908,11 +1021,11 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const GemmArgs 
         if constexpr (C::BLES == 2) {
           const int kr = 8 * half + ((lane & 15) >> 2);
           const int ch = (wn * C::WTN + 32 * j) / 8 + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1);
-          b_rd[j] = BM * RBA + kr * RBB + 16 * (ch ^ swz_tr<2, RBB>(kr)) + 8 * (lane & 1);
+          b_rd[j] = AREG + kr * RBB + 16 * (ch ^ swz_tr<2, RBB>(kr)) + 8 * (lane & 1);
         } else {
           const int kr = C::KPACK * half + ((lane & 15) >> 1);
           const int ch = (wn * C::WTN + 32 * j) / 16 + ((lane >> 4) & 1);
-          b_rd[j] = BM * RBA + kr * RBB + 16 * (ch ^ swz_tr<1, RBB>(kr)) + 8 * (lane & 1);
+          b_rd[j] = AREG + kr * RBB + 16 * (ch ^ swz_tr<1, RBB>(kr)) + 8 * (lane & 1);
         }
       }
     } else {
@@ -920,7 +1033,7 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const GemmArgs 
       for (int s = 0; s < S; ++s)
 #pragma unroll
         for (int q = 0; q < CPL; ++q)
-          b_rd[s * CPL + q] = BM * RBA + (wn * C::WTN + l32) * RBA + 16 * ((s * 2 * CPL + half * CPL + q) ^ swz_k128(l32));
+          b_rd[s * CPL + q] = AREG + (wn * C::WTN + l32) * RBB + 16 * ((s * 2 * CPL + half * CPL + q) ^ swz_k128(l32));
     }
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
 
@@ -934,10 +1047,24 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const GemmArgs 
       const uint32_t sb = lds0 + st * C::STAGE;
       static_for<0, C::TM>([&](auto ic) {
         constexpr int i = decltype(ic)::value;
-        if constexpr (CPL == 1) {
-          fa[SL][i] = lds_rd128<i * 32 * RBA>(sb + a_rd[SS][0]);
+        if constexpr (C::ATR) {
+          constexpr int O = SS * C::MK * RBA;
+          const uint32_t ad = sb + a_rd[i];
+          if constexpr (ES == 2) {
+            const u32x2v lo = lds_rd_tr16<O>(ad), hi = lds_rd_tr16<O + 4 * RBA>(ad);
+            fa[SL][i] = FT{lo.x, lo.y, hi.x, hi.y};
+          } else if constexpr (C::KPACK == 16) {
+            const u32x2v a = lds_rd_tr8<O>(ad), b = lds_rd_tr8<O + 8 * RBA>(ad);
+            fa[SL][i] = FT{a.x, a.y, b.x, b.y};
+          } else {
+            const u32x2v a = lds_rd_tr8<O>(ad), b = lds_rd_tr8<O + 8 * RBA>(ad), c = lds_rd_tr8<O + 16 * RBA>(ad),
+                         d = lds_rd_tr8<O + 24 * RBA>(ad);
+            fa[SL][i] = FT{a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y};
+          }
+        } else if constexpr (CPL == 1) {
+          fa[SL][i] = lds_rd128<i * 32 * RBA>(sb + a_rd[SS]);
         } else {
-          const u32x4 lo = lds_rd128<i * 32 * RBA>(sb + a_rd[SS][0]), hi = lds_rd128<i * 32 * RBA>(sb + a_rd[SS][1]);
+          const u32x4 lo = lds_rd128<i * 32 * RBA>(sb + a_rd[SS * CPL]), hi = lds_rd128<i * 32 * RBA>(sb + a_rd[SS * CPL + 1]);
           fa[SL][i] = FT{lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
         }
       });
@@ -964,7 +1091,7 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const GemmArgs 
               v = BF{a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y};
             }
           } else {
-            constexpr int O = j * 32 * RBA + bi * BREG;
+            constexpr int O = j * 32 * RBB + bi * BREG;
             if constexpr (CPL == 1) {
               v = lds_rd128<O>(sb + b_rd[SS * CPL]);
             } else {
@@ -979,7 +1106,8 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const GemmArgs 
     };
     // LDS read instructions per k-step (the wait count that leaves the next step's reads in flight)
     constexpr int BREADS = !C::BTR ? CPL : (C::BLES == 2 ? 2 : (BWIDEN ? 1 : C::KPACK / 8));
-    constexpr int NREAD = C::TM * CPL + C::TN * C::NB * BREADS;
+    constexpr int AREADS = !C::ATR ? CPL : (ES == 2 ? 2 : C::KPACK / 8);
+    constexpr int NREAD = C::TM * AREADS + C::TN * C::NB * BREADS;
     // (lgkmcnt counts to 15: with more reads per step the wait also covers some of the next step's reads)
     constexpr int NWAIT = NREAD < 15 ? NREAD : 15;
     // the reads into fragment slot SL are complete once at most N LDS reads are outstanding (N < 0: already waited
@@ -996,22 +1124,32 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const GemmArgs 
       }
     };
 
-    // prologue: tiles 0 (and 1 with three stages) in flight, tile 0 waited for
-    dma(0, 0);
-    if constexpr (NST == 3) {
-      if (KT > 1) {
-        dma(1, 1);
-        dma_barrier<OPS>();
-      } else {
-        dma_barrier<0>();
+    // tile kt complete, with the loads of at most min(ahead, NST - 2) later tiles still in flight
+    auto tile_barrier = [&](int ahead) {
+      if (NST > 2 && ahead >= NST - 2) dma_barrier<(NST - 2) * OPS>();
+      else if (NST == 4 && ahead == 1) dma_barrier<NST == 4 ? OPS : 0>();
+      else dma_barrier<0>();
+    };
+    // prologue: the first NST - 1 tiles in flight, tile 0 waited for
+    static_for<0, NST - 1>([&](auto tc) {
+      constexpr int t = decltype(tc)::value;
+      if (t < KT) {
+        before_dma(t);
+        dma(t, t);
       }
-    } else {
-      dma_barrier<0>();
+    });
+    tile_barrier(KT - 1);
+    if constexpr (EDGE) {
+      if (ktail < BK && kt0 == KTA - 1) zero_tail(0);
     }
     lfrag(0, int_c<0>{}, int_c<0>{});
     int cur = 0;
-    for (int kt = 0; kt < KT; ++kt) {
+    // one k-tile; LOAD: tile kt + NST - 1 is requested under its first k-step's MFMAs (a compile-time choice, so that
+    // the loads share the MFMAs' basic block and can be scheduled between them)
+    auto k_tile = [&](int kt, auto load) __attribute__((always_inline)) {
+      constexpr bool LOAD = decltype(load)::value;
       const int nxt = cur + 1 == NST ? 0 : cur + 1;
+      if constexpr (LOAD) before_dma(kt + NST - 1);
       static_for<0, S>([&](auto s) {
         constexpr int SS = decltype(s)::value;
         if constexpr (SS + 1 < S) {
@@ -1019,10 +1157,16 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const GemmArgs 
           wait_slot(int_c<SS & 1>{}, int_c<NWAIT>{});
         } else {
           // tile kt + 1 complete in every wave's LDS, and every wave done reading stage cur
-          if (NST == 3 && kt + 2 < KT) dma_barrier<NST == 3 ? OPS : 0>();
-          else dma_barrier<0>();
+          if constexpr (LOAD) dma_barrier<(NST - 2) * OPS>();
+          else if (kt + 1 < KT) tile_barrier(KT - 2 - kt);
+          else lgkm_wait<0>();
+          if constexpr (EDGE) {
+            if (ktail < BK && kt0 + kt + 1 == KTA - 1) zero_tail(nxt);
+          }
           wait_slot(int_c<SS & 1>{}, int_c<-1>{});
-          lfrag(nxt, int_c<0>{}, int_c<0>{});
+          // (nothing is read past the last tile: such a read, in flight when the loop ends, would land in registers
+          // that the compiler, which takes its output as written at once and never used, has given to the epilogue)
+          if (LOAD || kt + 1 < KT) lfrag(nxt, int_c<0>{}, int_c<0>{});
         }
         __builtin_amdgcn_sched_barrier(0);
         typename F::T wb[C::TN], wb2[DUAL ? C::TN : 1];
@@ -1043,22 +1187,23 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const GemmArgs 
             acc[i][j] = M::mma(wb[j], fa[SS & 1][i], acc[i][j]);
             if constexpr (DUAL) acc2[i][j] = M::mma(wb2[j], fa[SS & 1][i], acc2[i][j]);
           }
-        if constexpr (SS == 0) {
-          // tile kt + NST - 1 into the stage tile kt - 1 used (every wave finished reading it before the last barrier)
+        if constexpr (SS == 0 && LOAD) {
+          // into the stage tile kt - 1 used (every wave finished reading it before the last barrier)
           const int t = kt + NST - 1;
-          if (t < KT) {
-            dma(t, t % NST);
-            constexpr int NM = C::TM * C::TN * C::NB;
-            static_for<0, (OPS < NM ? OPS : NM)>([&](auto) {
-              __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
-              __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // VMEM read (DMA)
-            });
-          }
+          dma(t, NST == 4 ? (t & 3) : NST == 2 ? (t & 1) : t % NST);
+          constexpr int NM = C::TM * C::TN * C::NB;
+          static_for<0, (OPS < NM ? OPS : NM)>([&](auto) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
+            __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // VMEM read (DMA)
+          });
         }
         __builtin_amdgcn_sched_barrier(0);
       });
       cur = nxt;
-    }
+    };
+    int kt = 0;
+    for (; kt + NST - 1 < KT; ++kt) k_tile(kt, std::true_type{});
+    for (; kt < KT; ++kt) k_tile(kt, std::false_type{});
   } else {
     // One register stage of global prefetch: tile kt + 2 is requested at the start of k-tile kt (right after tile
     // kt + 1 went from registers to LDS), so each load has a whole k-tile of MFMA work to arrive in. Two LDS stages.
@@ -1275,18 +1420,21 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const GemmArgs 
     // moving the reads above the writes is all the ordering needed (a memory fence would also wait for the stores).
     __asm__ __volatile__("" ::: "memory");
     const int em0 = m0 + wm * C::WTM + round * EPI_ROWS * 32, en0 = n0 + wn * C::WTN;
-    if (G.splits > 1) {  // raw partial sums of this K range
-      constexpr int PDT = M::INT ? DT_S32 : DT_F32;
-      const int64_t slice = (int64_t)G.batch * G.M * G.N * 4;
-      char* ws = (char*)G.ws + (int64_t)split * C::NB * slice;
-      if (G.tile_counters) {  // read back by the range that finishes the tile: device-scope stores
-        epi_pass<EPI_STORE, PDT, M::INT, false, C::WTN, PITCH, EPI_ROWS * 32, false, true>(G, ws, b, em0, en0, patch,
-                                                                                          nullptr, lane);
-      } else {
-        epi_pass<EPI_STORE, PDT, M::INT, false, C::WTN, PITCH, EPI_ROWS * 32>(G, ws, b, em0, en0, patch, nullptr, lane);
-        if constexpr (DUAL)
-          epi_pass<EPI_STORE, PDT, M::INT, false, C::WTN, PITCH, EPI_ROWS * 32>(G, ws + slice, b, em0, en0,
-                                                                               patch + REGION, nullptr, lane);
+    if (C::SPLIT && G.splits > 1) {  // raw partial sums of this K range
+      if constexpr (C::SPLIT) {
+        constexpr int PDT = M::INT ? DT_S32 : DT_F32;
+        const int64_t slice = (int64_t)G.batch * G.M * G.N * 4;
+        char* ws = (char*)G.ws + (int64_t)split * C::NB * slice;
+        static_for<0, C::NB>([&](auto bc) {
+          constexpr int bi = decltype(bc)::value;
+          const uint32_t* reg = patch + bi * REGION;
+          if (G.tile_counters)  // read back by the range that finishes the tile: device-scope stores
+            epi_pass<EPI_STORE, PDT, M::INT, false, C::WTN, PITCH, EPI_ROWS * 32, EDGE, true>(G, ws + bi * slice, b, em0,
+                                                                                             en0, reg, nullptr, lane);
+          else
+            epi_pass<EPI_STORE, PDT, M::INT, false, C::WTN, PITCH, EPI_ROWS * 32, EDGE>(G, ws + bi * slice, b, em0, en0,
+                                                                                       reg, nullptr, lane);
+        });
       }
     } else {
       epi_round<M::INT, DUAL, C::WTN, PITCH, EPI_ROWS * 32, EDGE>(G, b, em0, en0, patch, patch + REGION, lane);
@@ -1298,7 +1446,7 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const GemmArgs 
   // counts its arrival at the tile; the last of the S ranges to arrive sums them all and applies the epilogue. No
   // workgroup waits for another, and no cache is flushed or invalidated (the partials are written and read at
   // device scope); the counter is back at zero when the launch ends.
-  if constexpr (!EDGE && !DUAL) {
+  if constexpr (C::SPLIT) {
     if (G.splits > 1 && G.tile_counters) {
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
@@ -1312,10 +1460,12 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const GemmArgs 
       __syncthreads();
       if (*(volatile int*)last) {
         switch (G.splits) {
-          case 2: splitk_finish_tile<M::INT, 2, BM, BN, C::THREADS>(G, b, m0, n0, tid); break;
-          case 4: splitk_finish_tile<M::INT, 4, BM, BN, C::THREADS>(G, b, m0, n0, tid); break;
-          case 8: splitk_finish_tile<M::INT, 8, BM, BN, C::THREADS>(G, b, m0, n0, tid); break;
-          case 16: splitk_finish_tile<M::INT, 16, BM, BN, C::THREADS>(G, b, m0, n0, tid); break;
+          case 2: splitk_finish_tile<M::INT, DUAL, EDGE, 2, BM, BN, C::THREADS>(G, b, m0, n0, tid); break;
+          case 4: splitk_finish_tile<M::INT, DUAL, EDGE, 4, BM, BN, C::THREADS>(G, b, m0, n0, tid); break;
+          case 8: splitk_finish_tile<M::INT, DUAL, EDGE, 8, BM, BN, C::THREADS>(G, b, m0, n0, tid); break;
+          case 16:
+            if constexpr (!DUAL) splitk_finish_tile<M::INT, DUAL, EDGE, 16, BM, BN, C::THREADS>(G, b, m0, n0, tid);
+            break;
         }
       }
     }
@@ -1356,16 +1506,31 @@ Choice edge_choice(bool ar, bool br, const char* name) {
   return br ? make_choice<KIND, BM, BN, BK, WM, WN, false, true, DUAL, true>(name)
             : make_choice<KIND, BM, BN, BK, WM, WN, false, false, DUAL, true>(name);
 }
+// The same for tiles of fewer than 64 rows, which exist for a K-contiguous A only (an m-contiguous one would have LDS
+// rows shorter than the transposing reads take).
+template <int KIND, int BM, int BN, int BK, int WM, int WN, bool DUAL>
+Choice edge_choice_k(bool br, const char* name) {
+  return br ? make_choice<KIND, BM, BN, BK, WM, WN, false, true, DUAL, true>(name)
+            : make_choice<KIND, BM, BN, BK, WM, WN, false, false, DUAL, true>(name);
+}
 
-// Per-type instantiation pickers (one translation unit each, so the build parallelises). `ar`: A is m-contiguous,
-// `br`: B is n-contiguous. Tile-multiple shapes with a K-contiguous A get the full-tile kernels; any other shape (and
-// an m-contiguous A) gets the edge kernel of a 128×128 tile (64×64 for f32). With g.splits > 1 a picker returns the
-// tile it runs over each of the K ranges, or false (split-K runs full tiles only).
+// Per-type instantiation pickers (several translation units, so the build parallelises). `ar`: A is m-contiguous, `br`:
+// B is n-contiguous. pick_*: multiples of 128 rows and columns (64 for f32) with a K-contiguous A get the full-tile
+// kernels; false for any other shape. With g.splits > 1 a picker returns the tile it runs over each of the K ranges, or
+// false. edge_tiles_*: the edge kernels of such other shapes, in `c` (room for 4); pick_edge_tile takes the one whose
+// time it estimates lowest.
 bool pick_bf16(const GemmArgs& g, bool ar, bool br, Choice* c);
 bool pick_f16(const GemmArgs& g, bool ar, bool br, Choice* c);
 bool pick_i8(const GemmArgs& g, bool ar, bool br, Choice* c);
 bool pick_fp8(const GemmArgs& g, bool ar, bool br, Choice* c);
 bool pick_f32(const GemmArgs& g, bool ar, bool br, Choice* c);
 bool pick_bf16f8(const GemmArgs& g, bool ar, bool br, Choice* c);
+int edge_tiles_bf16(const GemmArgs& g, bool ar, bool br, Choice* c);
+int edge_tiles_f16(const GemmArgs& g, bool ar, bool br, Choice* c);
+int edge_tiles_i8(const GemmArgs& g, bool ar, bool br, Choice* c);
+int edge_tiles_fp8(const GemmArgs& g, bool ar, bool br, Choice* c);
+int edge_tiles_f32(const GemmArgs& g, bool ar, bool br, Choice* c);
+int edge_tiles_bf16f8(const GemmArgs& g, bool ar, bool br, Choice* c);
+int edge_tiles_bf16f8_dual(const GemmArgs& g, bool ar, bool br, Choice* c);
 
 }  // namespace ryft

@@ -1,4 +1,4 @@
-// MFMA GEMM instantiations: bf16, f16.
+// MFMA GEMM instantiations: bf16, full tiles.
 #include "gemm_mfma.h"
 
 namespace ryft {
@@ -13,6 +13,13 @@ bool pick_bf16(const GemmArgs& g, bool ar, bool br, Choice* c) {
     return true;
   }
   const int64_t tiles256 = (int64_t)(g.M / 256) * (g.N / 256) * g.batch;
+  if (fits(256, 256, 64) && tiles256 >= 128 && tiles256 < 192) {
+    // 256×256 tiles that would leave a quarter of the CUs or more idle: twice as many of half the size
+    // (2048 × 4096 × 4096: 128 tiles of 256×256 take 84 µs, 256 of 256×128 59 µs)
+    *c = br ? make_choice<MMA_BF16, 256, 128, 64, 4, 2, false, true, false>("gemm_bf16_mfma_256x128")
+            : make_choice<MMA_BF16, 256, 128, 64, 4, 2, false, false, false>("gemm_bf16_mfma_256x128");
+    return true;
+  }
   if (fits(256, 256, 64) && tiles256 >= 128) {
     // eight waves (two per SIMD, 128×64 each): one wave's LDS waits and barrier overlap the other's MFMAs
     *c = br ? make_choice<MMA_BF16, 256, 256, 64, 2, 4, false, true, false>("gemm_bf16_mfma_256x256")
@@ -24,21 +31,7 @@ bool pick_bf16(const GemmArgs& g, bool ar, bool br, Choice* c) {
             : make_choice<MMA_BF16, 128, 128, 64, 2, 2, false, false, false>("gemm_bf16_mfma_128x128");
     return true;
   }
-  *c = edge_choice<MMA_BF16, 128, 128, 64, 2, 2, false>(ar, br, "gemm_bf16_mfma_edge_128x128");
-  return true;
-}
-
-bool pick_f16(const GemmArgs& g, bool ar, bool br, Choice* c) {
-  auto fits = [&](int bm, int bn, int bk) { return !ar && g.M % bm == 0 && g.N % bn == 0 && g.K % bk == 0; };
-  if (g.dual) return false;
-  if (fits(128, 128, 64 * (g.splits > 1 ? g.splits : 1))) {
-    *c = br ? make_choice<MMA_F16, 128, 128, 64, 2, 2, false, true, false>("gemm_f16_mfma_128x128")
-            : make_choice<MMA_F16, 128, 128, 64, 2, 2, false, false, false>("gemm_f16_mfma_128x128");
-    return true;
-  }
-  if (g.splits > 1) return false;
-  *c = edge_choice<MMA_F16, 128, 128, 64, 2, 2, false>(ar, br, "gemm_f16_mfma_edge_128x128");
-  return true;
+  return false;
 }
 
 }  // namespace ryft

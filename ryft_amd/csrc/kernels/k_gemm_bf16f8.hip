@@ -1,4 +1,4 @@
-// MFMA GEMM instantiations: bf16 activations × f8E4M3FN weights (an n-contiguous B stays f8 in LDS and is widened to
+// MFMA GEMM instantiations: bf16 activations × f8E4M3FN weights, full tiles (an n-contiguous B stays f8 in LDS and is widened to
 // bf16 in registers after its transposing read; a K-contiguous B is widened on its way into LDS).
 #include "gemm_mfma.h"
 
@@ -30,8 +30,7 @@ bool pick_bf16f8(const GemmArgs& g, bool ar, bool br, Choice* c) {
               : make_choice<MMA_BF16_F8, 128, 128, 64, 2, 2, false, false, true>("gemm_bf16f8_mfma_dual_128x128");
       return true;
     }
-    *c = edge_choice<MMA_BF16_F8, 128, 128, 64, 2, 2, true>(ar, br, "gemm_bf16f8_mfma_dual_edge_128x128");
-    return true;
+    return false;
   }
   const int64_t tiles256 = (int64_t)(g.M / 256) * (g.N / 256) * g.batch;
   if (fits(256, 256, 64) && tiles256 >= 128) {
@@ -44,8 +43,7 @@ bool pick_bf16f8(const GemmArgs& g, bool ar, bool br, Choice* c) {
             : make_choice<MMA_BF16_F8, 128, 128, 64, 2, 2, false, false, false>("gemm_bf16f8_mfma_128x128");
     return true;
   }
-  *c = edge_choice<MMA_BF16_F8, 128, 128, 64, 2, 2, false>(ar, br, "gemm_bf16f8_mfma_edge_128x128");
-  return true;
+  return false;
 }
 
 }  // namespace ryft

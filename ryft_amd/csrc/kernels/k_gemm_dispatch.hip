@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <string>
 #include <type_traits>
 
@@ -186,6 +187,86 @@ static unsigned layout_gaps(const GemmArgs& g, int kind, int* ar, int* br) {
   return gaps;
 }
 
+// The full-tile kernel of these arguments, if their shape has one.
+static bool pick_full(const GemmArgs& g, int kind, bool ar, bool br, Choice* c) {
+  switch (kind) {
+    case MMA_BF16: return pick_bf16(g, ar, br, c);
+    case MMA_F16: return pick_f16(g, ar, br, c);
+    case MMA_I8: return pick_i8(g, ar, br, c);
+    case MMA_FP8: return pick_fp8(g, ar, br, c);
+    case MMA_F32: return pick_f32(g, ar, br, c);
+    case MMA_BF16_F8: return pick_bf16f8(g, ar, br, c);
+    default: return false;
+  }
+}
+
+// Whether an edge tile can run its K in `splits` ranges: whole octets per row for the finish, a tile that has the split
+// compiled in (at most 16 ranges, 8 of a dual GEMM), and no empty range.
+static bool edge_splittable(const GemmArgs& g, const Choice& c, int splits) {
+  const int kt = (g.K + c.bk - 1) / c.bk, per = (kt + splits - 1) / splits;
+  return g.N % 8 == 0 && c.bm * c.bn * (g.dual ? 2 : 1) <= 128 * 256 && splits <= (g.dual ? 8 : 16) &&
+         (int64_t)(splits - 1) * per < kt;
+}
+
+// Microseconds of one k-tile (128 bytes of k per row; 64 for f32) of an edge tile: `alone`, of a workgroup with a CU to
+// itself, and `shared`, per workgroup of a busy CU. Measured at (M, K, N) = (1, 4096, 4096), (16, 4096, 14336),
+// (64, 4096, 4096), (300, 4096, 8192), (1000, 1000, 1000), (2000, 3000, 4000) and others, every tile and split of each:
+// small tiles move more operand bytes per product (a 64×64 tile's k-tile takes 0.27 µs whether the CU runs one or eight
+// of them: it is the L2-to-LDS rate, about 60 GB/s per CU) but there are more of them to fill the chip with.
+struct TileTime {
+  int kind, bm, bn, dual;
+  double alone, shared;
+};
+static constexpr TileTime kTileTimes[] = {
+    {MMA_BF16, 256, 256, 0, 1.4, 1.95},    {MMA_BF16, 128, 128, 0, 0.77, 0.56},   {MMA_BF16, 64, 64, 0, 0.27, 0.27},
+    {MMA_BF16, 32, 128, 0, 0.29, 0.275},   {MMA_F16, 128, 128, 0, 0.77, 0.56},    {MMA_I8, 256, 256, 0, 1.4, 2.0},
+    {MMA_I8, 128, 128, 0, 0.9, 0.7},       {MMA_I8, 64, 128, 0, 0.45, 0.42},      {MMA_I8, 32, 128, 0, 0.3, 0.27},
+    {MMA_FP8, 128, 128, 0, 0.9, 0.7},      {MMA_FP8, 128, 128, 1, 1.4, 1.0},      {MMA_F32, 64, 64, 0, 0.45, 0.38},
+    {MMA_BF16_F8, 128, 128, 0, 0.9, 0.46}, {MMA_BF16_F8, 64, 128, 0, 0.38, 0.24}, {MMA_BF16_F8, 32, 128, 0, 0.28, 0.18},
+    {MMA_BF16_F8, 128, 128, 1, 1.3, 1.0},  {MMA_BF16_F8, 64, 128, 1, 0.66, 0.65}, {MMA_BF16_F8, 32, 128, 1, 0.6, 0.34}};
+
+// Estimated microseconds of an edge tile over `splits` K ranges: the k-tiles of the busiest CU's workgroups, and for a
+// split the arrival and finish in-kernel (partial sums up to 8 MiB) or the reduction launch, both growing with the
+// partial sums' traffic.
+static double edge_cost(const GemmArgs& g, int kind, const Choice& c, int splits) {
+  const TileTime* t = nullptr;
+  for (const TileTime& x : kTileTimes)
+    if (x.kind == kind && x.bm == c.bm && x.bn == c.bn && x.dual == (g.dual ? 1 : 0)) t = &x;
+  const double wgs = (double)((g.M + c.bm - 1) / c.bm) * ((g.N + c.bn - 1) / c.bn) * g.batch * splits;
+  const int kt = (g.K + c.bk - 1) / c.bk, per = (kt + splits - 1) / splits;
+  // (a chip full of single workgroups runs at the shared rate already where that is the slower one)
+  const double each = t ? (wgs <= 192 ? t->alone : std::max(t->alone, t->shared * std::ceil(wgs / 256))) : wgs;
+  double us = 3.0 + per * each;
+  if (splits > 1) {
+    const double mb = (double)splits * (g.dual ? 2 : 1) * g.batch * g.M * g.N * 4.0 / (1 << 20);
+    us += mb <= 8.0 ? 3.0 + 0.5 * mb : 5.5 + 0.55 * mb;
+  }
+  return us;
+}
+
+// The edge kernel for these arguments (g.splits K ranges): the candidate whose estimated time is lowest.
+static bool pick_edge_tile(const GemmArgs& g, int kind, bool ar, bool br, Choice* c) {
+  Choice t[4];
+  int n = 0;
+  switch (kind) {
+    case MMA_BF16: n = edge_tiles_bf16(g, ar, br, t); break;
+    case MMA_F16: n = edge_tiles_f16(g, ar, br, t); break;
+    case MMA_I8: n = edge_tiles_i8(g, ar, br, t); break;
+    case MMA_FP8: n = edge_tiles_fp8(g, ar, br, t); break;
+    case MMA_F32: n = edge_tiles_f32(g, ar, br, t); break;
+    case MMA_BF16_F8: n = edge_tiles_bf16f8(g, ar, br, t); break;
+  }
+  int best = -1;
+  const int splits = std::max(1, (int)g.splits);
+  for (int i = 0; i < n; ++i) {
+    if (g.splits > 1 && !edge_splittable(g, t[i], g.splits)) continue;
+    if (best < 0 || edge_cost(g, kind, t[i], splits) < edge_cost(g, kind, t[best], splits)) best = i;
+  }
+  if (best < 0) return false;
+  *c = t[best];
+  return true;
+}
+
 // Returns true and fills `c` when an MFMA instantiation covers these arguments.
 static bool pick_mfma(const GemmArgs& g, Choice* c) {
   // MFMA epilogues implement store / scale / SwiGLU; generic programs run on the generic kernel
@@ -203,15 +284,11 @@ static bool pick_mfma(const GemmArgs& g, Choice* c) {
   const int bes = kind == MMA_BF16_F8 ? 1 : es;  // B's element size in HBM
   int ar = 0, br = 0;
   if (layout_gaps(g, kind, &ar, &br)) return false;
-  bool ok = false;
-  switch (kind) {
-    case MMA_BF16: ok = pick_bf16(g, ar, br, c); break;
-    case MMA_F16: ok = pick_f16(g, ar, br, c); break;
-    case MMA_I8: ok = pick_i8(g, ar, br, c); break;
-    case MMA_FP8: ok = pick_fp8(g, ar, br, c); break;
-    case MMA_F32: ok = pick_f32(g, ar, br, c); break;
-    case MMA_BF16_F8: ok = pick_bf16f8(g, ar, br, c); break;
-  }
+  bool ok = pick_full(g, kind, ar, br, c);
+  // (shapes that run full tiles are split over full tiles or not at all)
+  GemmArgs whole = g;
+  whole.splits = 1;
+  if (!ok && !(g.splits > 1 && pick_full(whole, kind, ar, br, c))) ok = pick_edge_tile(g, kind, ar, br, c);
   if (ok && c->edge) {
     // the edge kernels zero k positions past K a load at a time: K must end on a load boundary of each
     // K-contiguous operand (16-byte vectors; 8-byte pieces for a widened f8 B)
@@ -247,11 +324,31 @@ const char* gemm_kernel_name(const GemmArgs& a) {
   return "gemm_generic";
 }
 
+bool gemm_edge_tile(const GemmArgs& a, int* bm, int* bn) {
+  Choice c;
+  if (!pick_mfma(a, &c) || !c.edge) return false;
+  *bm = c.bm;
+  *bn = c.bn;
+  return true;
+}
+
 int gemm_plan_splits(const GemmArgs& a) {
   GemmArgs g = a;
   g.splits = 1;
   Choice c;
   if (!pick_mfma(g, &c)) return 1;
+  if (c.edge) {
+    int best = 1;
+    const int kind = mma_kind(g);
+    double cost = edge_cost(g, kind, c, 1);
+    for (int s = 2; s <= 16; s *= 2) {
+      g.splits = s;
+      if (!pick_mfma(g, &c)) continue;
+      const double t = edge_cost(g, kind, c, s);
+      if (t < cost) best = s, cost = t;
+    }
+    return best;
+  }
   const int64_t tiles = (int64_t)((g.M + c.bm - 1) / c.bm) * ((g.N + c.bn - 1) / c.bn) * g.batch;
   const bool f32 = g.A.dtype == DT_F32;
   // the 64-row tile (chosen when 128×128 tiles would not cover the chip) reads twice the operand bytes per FLOP of a
@@ -287,10 +384,10 @@ void launch_gemm(const GemmArgs& g, hipStream_t stream, hipEvent_t done) {
       if (e != hipSuccess) fail(PJRT_Error_Code_INTERNAL, std::string("LDS attribute failed: ") + hipGetErrorString(e));
     }
     const int splits = g.splits > 1 ? g.splits : 1;
-    if (splits > 1 && (!g.ws || g.K % (splits * 16) || g.N % 16 || c.edge))
-      fail(PJRT_Error_Code_INTERNAL, "split-K without a workspace, on partial tiles or with N not a multiple of 16");
-    if (splits > 1 && g.tile_counters && (g.dual || (splits & (splits - 1)) || splits > 16))
-      fail(PJRT_Error_Code_INTERNAL, "in-kernel split-K finish for a dual GEMM or " + std::to_string(splits) + " ranges");
+    if (splits > 1 && (!g.ws || (c.edge ? !edge_splittable(g, c, splits) : g.K % (splits * 16) || g.N % 16)))
+      fail(PJRT_Error_Code_INTERNAL, "split-K without a workspace or over partial ranges");
+    if (splits > 1 && g.tile_counters && ((g.dual && (!c.edge || splits > 8)) || (splits & (splits - 1)) || splits > 16))
+      fail(PJRT_Error_Code_INTERNAL, "in-kernel split-K finish of " + std::to_string(splits) + " ranges");
     int64_t blocks = (int64_t)((g.M + c.bm - 1) / c.bm) * ((g.N + c.bn - 1) / c.bn) * g.batch * splits;
     if (blocks > INT32_MAX) fail(PJRT_Error_Code_UNIMPLEMENTED, "too many GEMM tiles");
     void* args[] = {(void*)&g};

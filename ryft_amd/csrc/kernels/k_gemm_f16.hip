@@ -1,0 +1,23 @@
+// MFMA GEMM instantiations: f16.
+#include "gemm_mfma.h"
+
+namespace ryft {
+
+bool pick_f16(const GemmArgs& g, bool ar, bool br, Choice* c) {
+  auto fits = [&](int bm, int bn, int bk) { return !ar && g.M % bm == 0 && g.N % bn == 0 && g.K % bk == 0; };
+  if (g.dual) return false;
+  if (fits(128, 128, 64 * (g.splits > 1 ? g.splits : 1))) {
+    *c = br ? make_choice<MMA_F16, 128, 128, 64, 2, 2, false, true, false>("gemm_f16_mfma_128x128")
+            : make_choice<MMA_F16, 128, 128, 64, 2, 2, false, false, false>("gemm_f16_mfma_128x128");
+    return true;
+  }
+  return false;
+}
+
+int edge_tiles_f16(const GemmArgs& g, bool ar, bool br, Choice* c) {
+  if (g.dual) return 0;
+  c[0] = edge_choice<MMA_F16, 128, 128, 64, 2, 2, false>(ar, br, "gemm_f16_mfma_edge_128x128");
+  return 1;
+}
+
+}  // namespace ryft

@@ -11,9 +11,13 @@ bool pick_f32(const GemmArgs& g, bool ar, bool br, Choice* c) {
             : make_choice<MMA_F32, 64, 64, 16, 2, 2, false, false, false>("gemm_f32_mfma_64x64");
     return true;
   }
-  if (g.splits > 1) return false;
-  *c = edge_choice<MMA_F32, 64, 64, 16, 2, 2, false>(ar, br, "gemm_f32_mfma_edge_64x64");
-  return true;
+  return false;
+}
+
+int edge_tiles_f32(const GemmArgs& g, bool ar, bool br, Choice* c) {
+  if (g.dual) return 0;
+  c[0] = edge_choice<MMA_F32, 64, 64, 16, 2, 2, false>(ar, br, "gemm_f32_mfma_edge_64x64");
+  return 1;
 }
 
 }  // namespace ryft

@@ -12,10 +12,7 @@ bool pick_fp8(const GemmArgs& g, bool ar, bool br, Choice* c) {
     return true;
   }
   if (g.dual) {
-    if (!fits(128, 128, 128)) {
-      *c = edge_choice<MMA_FP8, 128, 128, 128, 2, 2, true>(ar, br, "gemm_fp8_mfma_dual_edge_128x128");
-      return true;
-    }
+    if (!fits(128, 128, 128)) return false;
     *c = br ? make_choice<MMA_FP8, 128, 128, 128, 2, 2, false, true, true>("gemm_fp8_mfma_dual_128x128")
             : make_choice<MMA_FP8, 128, 128, 128, 2, 2, false, false, true>("gemm_fp8_mfma_dual_128x128");
     return true;
@@ -30,8 +27,13 @@ bool pick_fp8(const GemmArgs& g, bool ar, bool br, Choice* c) {
             : make_choice<MMA_FP8, 64, 128, 128, 2, 2, false, false, false>("gemm_fp8_mfma_64x128");
     return true;
   }
-  *c = edge_choice<MMA_FP8, 128, 128, 128, 2, 2, false>(ar, br, "gemm_fp8_mfma_edge_128x128");
-  return true;
+  return false;
+}
+
+int edge_tiles_fp8(const GemmArgs& g, bool ar, bool br, Choice* c) {
+  c[0] = g.dual ? edge_choice<MMA_FP8, 128, 128, 128, 2, 2, true>(ar, br, "gemm_fp8_mfma_dual_edge_128x128")
+                : edge_choice<MMA_FP8, 128, 128, 128, 2, 2, false>(ar, br, "gemm_fp8_mfma_edge_128x128");
+  return 1;
 }
 
 }  // namespace ryft

@@ -1,4 +1,4 @@
-// MFMA GEMM instantiations: i8.
+// MFMA GEMM instantiations: i8, full tiles.
 #include "gemm_mfma.h"
 
 namespace ryft {
@@ -24,8 +24,7 @@ bool pick_i8(const GemmArgs& g, bool ar, bool br, Choice* c) {
             : make_choice<MMA_I8, 128, 128, 128, 2, 2, false, false, false>("gemm_i8_mfma_128x128");
     return true;
   }
-  *c = edge_choice<MMA_I8, 128, 128, 128, 2, 2, false>(ar, br, "gemm_i8_mfma_edge_128x128");
-  return true;
+  return false;
 }
 
 }  // namespace ryft

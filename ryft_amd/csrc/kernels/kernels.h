@@ -28,6 +28,8 @@ void launch_scatter(const ScatterArgs& a, hipStream_t stream, hipEvent_t done = 
 int gemm_mfma_layout_gaps(const GemmArgs& a);
 // Name of the GEMM kernel launch_gemm() picks for these arguments (used for profiling labels).
 const char* gemm_kernel_name(const GemmArgs& a);
+// Whether launch_gemm() runs these arguments on an edge kernel (its name stands for the family), and on which tile.
+bool gemm_edge_tile(const GemmArgs& a, int* bm, int* bn);
 // Number of K ranges launch_gemm splits these arguments into when given a workspace of
 // splits × (dual ? 2 : 1) × batch × M × N 4-byte accumulators (1: no split).
 int gemm_plan_splits(const GemmArgs& a);

@@ -1900,18 +1900,23 @@ void Planner::plan_split_k(Step& st) {
   // their whole traffic then stays short of the tail a reduction launch adds (C1: 2 MiB, 11.2 against 13.5 µs a
   // step). Large ones (C5's down projection: 32 MiB) go to the reduction launch, which reads them with every CU
   // instead of one finishing workgroup per tile (75 against 89 µs).
-  const double partial_bytes = (double)s * G.batch * G.M * G.N * 4.0;
-  if (!G.dual && partial_bytes <= 8.0 * (1 << 20)) {
+  const double partial_bytes = (double)s * (G.dual ? 2 : 1) * G.batch * G.M * G.N * 4.0;
+  int bm = 0, bn = 0;
+  const bool edge = gemm_edge_tile(G, &bm, &bn);
+  if ((!G.dual || edge) && partial_bytes <= 8.0 * (1 << 20)) {
     // per-output-tile arrival counters for the in-kernel finish: part of the executable (zeroed once when it is
-    // loaded; each launch leaves them at zero), sized for the smallest tile any split kernel uses (64×64)
+    // loaded; each launch leaves them at zero), sized for the edge kernel's tile, or for the smallest full tile any
+    // split kernel uses (64×64)
     TensorType ct;
     ct.dtype = DType::S32;
-    ct.shape = {(int64_t)G.batch * ((G.M + 63) / 64) * ((G.N + 63) / 64)};
+    if (!edge) bm = bn = 64;
+    ct.shape = {(int64_t)G.batch * ((G.M + bm - 1) / bm) * ((G.N + bn - 1) / bn)};
     const int cs = new_slot(Slot::CONSTANT, ct);
     plan_.slots[cs].literal.assign((size_t)ct.bytes(), 0);
     st.patches.push_back({offsetof(GemmArgs, tile_counters), cs});
   }
-  st.name = std::string(gemm_kernel_name(G)) + "_splitk" + std::to_string(s);
+  // (an edge kernel's label names its family; the plan's text gives the tile and the ranges)
+  st.name = edge ? gemm_kernel_name(G) : std::string(gemm_kernel_name(G)) + "_splitk" + std::to_string(s);
 }
 
 // Replace a generic epilogue program by a specialised epilogue when its expression has one of the shapes the GEMM
@@ -2412,6 +2417,9 @@ std::string Plan::describe() const {
          << " out=" << dtype_name((DType)g.out_dtype[0]);
       if (g.raw_out) os << "+" << dtype_name((DType)g.out_dtype[1]);
       if (g.mid_round) os << " mid_round=" << dtype_name((DType)g.mid_round);
+      int bm, bn;
+      if (gemm_edge_tile(g, &bm, &bn)) os << " tile=" << bm << "x" << bn;
+      if (g.splits > 1) os << " splits=" << g.splits;
     } else if (s.kind == Step::ELEMENTWISE) {
       os << " instrs=" << s.ew.n_instr << " leaves=" << s.ew.n_leaves << " elems=" << s.ew.total;
     } else if (s.kind == Step::REDUCE) {

@@ -1,0 +1,77 @@
+"""The edge GEMM tiles (256×256 down to 32×128) and their K ranges against the oracle, at the sizes where they can go
+wrong: one row, one past and one short of a tile, k tails of one vector, ranges of unequal length, both layouts of
+each operand, dual GEMMs finished from partial sums.
+
+Tolerances: f32 accumulation of n products is off by at most n·2^-24 relative to the sum of magnitudes, and bf16 results
+by 2^-9, taken as 2^-7 for both sides and cancellation; integers exactly."""
+import pytest
+
+from edge_programs import dot
+from helpers import check, oracle_outputs, run_pjrt
+from ryft_amd import configs
+
+pytestmark = pytest.mark.gpu
+BF16 = 2.0 ** -7
+
+CASES = [
+    # (program, tile, split over K)
+    (dot("bf16_one_row", (1, 4096), (4096, 1032), "bf16", "f32", [1], [0], seed=31), "32x128", True),
+    (dot("bf16_33_rows", (33, 1096), (1096, 2056), "bf16", "f32", [1], [0], seed=32), None, False),
+    (dot("bf16_64_tiles", (1000, 1000), (1000, 1000), "bf16", "f32", [1], [0], seed=33), "64x64", False),
+    (dot("bf16_k_contiguous_both", (65, 2056), (1031, 2056), "bf16", "f32", [1], [1], seed=34), None, False),
+    (dot("bf16_m_contiguous_tail", (1001, 136), (1001, 264), "bf16", "f32", [0], [0], seed=35), None, True),
+    (dot("bf16_128_tiles", (2000, 520), (520, 2056), "bf16", "f32", [1], [0], seed=36), "128x128", False),
+    (dot("bf16_256_tiles", (136, 4088), (136, 4088), "bf16", "f32", [0], [0], seed=37), "256x256", False),
+    (dot("bf16_256_tiles_k_contiguous_b", (72, 4096), (4088, 72), "bf16", "f32", [0], [1], seed=38), "256x256", False),
+    (dot("i8_one_row", (1, 4096), (4096, 2064), "i8", "i32", [1], [0], seed=39), "32x128", True),
+    (dot("i8_rows_of_tiles", (129, 528), (528, 1040), "i8", "i32", [1], [0], seed=40), None, False),
+    (dot("i8_k_contiguous_both", (250, 1040), (263, 1040), "i8", "i32", [1], [1], seed=41), None, False),
+    (dot("i8_m_contiguous", (528, 272), (528, 144), "i8", "i32", [0], [0], seed=42), None, False),
+    (dot("f32_ranges", (33, 1000), (1000, 264), "f32", "f32", [1], [0], seed=43), "64x64", True),
+    (dot("f16_tail", (130, 264), (264, 136), "f16", "f32", [1], [0], seed=44), "128x128", False),
+    (dot("fp8_tail", (130, 272), (272, 144), "f8E4M3FN", "f32", [1], [0], seed=45), "128x128", False),
+    (dot("fp8_m_contiguous", (272, 144), (272, 144), "f8E4M3FN", "f32", [0], [0], seed=46), "128x128", False),
+]
+
+
+@pytest.mark.parametrize("case", CASES, ids=[c[0][0] for c in CASES])
+def test_gemm_tiles(gpu_client, case):
+    (name, prog, ins), tile, split = case
+    outs, exe = run_pjrt(gpu_client, prog, ins)
+    plan = exe.describe_plan()
+    assert "_edge_" in plan and (tile is None or f"tile={tile}" in plan), plan
+    assert not split or "splits=" in plan, plan
+    err = check(outs[0], oracle_outputs(prog, ins)[0], BF16, name)
+    again, _ = run_pjrt(gpu_client, prog, ins, executable=exe)
+    assert (outs[0] == again[0]).all()
+    print(f"[tiles] {name} {plan.splitlines()[-1].split('tile=')[1].split(' flops')[0]} error {err:.2e}", flush=True)
+
+
+@pytest.mark.parametrize("kw", [dict(m=1, d=1024, f=2048), dict(m=16, d=2048, f=1040), dict(m=33, d=1040, f=2048),
+                                dict(m=77, d=1280, f=2048), dict(m=130, d=512, f=528)])
+def test_swiglu_of_few_rows(gpu_client, kw):
+    # the dual gate / up GEMM and the down projection of a few rows: 32-row tiles, partial sums of both accumulators
+    w = configs.c5_swiglu_fp8(**kw)
+    outs, exe = run_pjrt(gpu_client, w.program, w.inputs)
+    assert "gemm_bf16f8_mfma_dual_edge" in exe.describe_plan()
+    # three bf16 roundings in a row (norm, SwiGLU product, result), on both sides
+    err = check(outs[0], oracle_outputs(w.program, w.inputs)[0], 3 * 2.0 ** -8, str(kw))
+    again, _ = run_pjrt(gpu_client, w.program, w.inputs, executable=exe)
+    assert (outs[0] == again[0]).all()
+    print(f"[tiles] swiglu {kw} error {err:.2e}", flush=True)
+
+
+def test_infinities_past_the_last_k_stay_out(gpu_client):
+    """A partial last k-tile reads the last valid k again and zeroes it: an infinity there is multiplied once, not by
+    the zeros of the padding (0 · inf would turn the result into NaN)."""
+    import numpy as np
+    from oracle import stablehlo as sh
+    for spec in (((9, 72), (72, 24), [1], [0]), ((72, 16), (72, 24), [0], [0]), ((9, 72), (25, 72), [1], [1])):
+        name, prog, ins = dot("inf_tail", spec[0], spec[1], "bf16", "f32", spec[2], spec[3], seed=47)
+        last = [slice(None)] * 2
+        last[spec[3][0]] = -1
+        ins[1].data[tuple(last)] = 0x7F80  # +inf at k = 71
+        outs, exe = run_pjrt(gpu_client, prog, ins)
+        (want, dt), = oracle_outputs(prog, ins)
+        got = sh.from_raw(outs[0], dt)
+        assert np.isinf(want).all() and (got == want).all()
