@@ -304,6 +304,18 @@ struct GatherArgs {
   int64_t total;       // result elements
 };
 
+// ------------------------------------------------------------------------------------------------ operand packing
+// A dot operand whose rows the MFMA loads cannot read, copied to dst[batch][k][pitch], its free dimension contiguous:
+// dst[b][k][f] = src[b·sb + k·sk + f·sf] for f < F (pitch: F rounded up to 16 elements; the rest is unspecified).
+struct PackArgs {
+  const void* src;
+  void* dst;
+  int64_t sb, sk, sf;  // element strides of the source
+  int32_t batch, K, F, pitch;
+  int32_t elem_bytes;  // 1, 2 or 4
+  int32_t pad_;
+};
+
 // ------------------------------------------------------------------------------------------------ scatter
 enum ScatterKind : int32_t { SC_SET = 0, SC_ADD = 1, SC_MUL = 2, SC_MIN = 3, SC_MAX = 4, SC_AND = 5, SC_OR = 6 };
 

@@ -6,6 +6,7 @@
 // vectors in both tensors, one element per thread otherwise. Memory-bound byte moves; no arithmetic on the values.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <string>
 
 #include "../common.h"
@@ -451,6 +452,118 @@ void launch_scatter(const ScatterArgs& a, hipStream_t stream, hipEvent_t done) {
     case 8: return launch_scatter_es<8>(a, stream, done);
     default: fail(PJRT_Error_Code_INTERNAL, "scatter element size " + std::to_string(a.elem_bytes));
   }
+}
+
+// ------------------------------------------------------------------------------------------------ operand packing
+namespace {
+
+// 16 bytes from any address (gfx950 reads unaligned vectors; the compiler is told nothing about the alignment).
+__device__ __forceinline__ u32x4w load_unaligned16(const char* p) {
+  u32x4w v;
+  __builtin_memcpy(&v, p, 16);
+  return v;
+}
+
+template <int ES> struct PackElem { using T = uint32_t; };
+template <> struct PackElem<1> { using T = uint8_t; };
+template <> struct PackElem<2> { using T = uint16_t; };
+
+// Rows that only need another pitch (sf == 1), or, gathered element by element, any strides: a 16-byte chunk of the
+// result per thread. HBM-bound; a row's last chunk is read element by element, so that nothing past it is touched.
+// 4 × [3216, 1812] bf16: 233 µs with its product when the elementwise interpreter copied it an element at a time, 34 now.
+template <int ES>
+__global__ void __launch_bounds__(256) pack_rows_kernel(const PackArgs A) {
+  using T = typename PackElem<ES>::T;
+  constexpr int V = 16 / ES;
+  const uint32_t cpr = (uint32_t)A.pitch / V, total = (uint32_t)A.K * cpr;
+  for (int b = blockIdx.y; b < A.batch; b += gridDim.y)
+    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < total; i += gridDim.x * 256) {
+      const uint32_t k = i / cpr, f0 = (i - k * cpr) * V;
+      const T* src = (const T*)A.src + (int64_t)b * A.sb + (int64_t)k * A.sk + (int64_t)f0 * A.sf;
+      u32x4w v = u32x4w{0, 0, 0, 0};
+      if (A.sf == 1 && (int)f0 + V <= A.F) {
+        v = load_unaligned16((const char*)src);
+      } else {
+        T e[V];
+#pragma unroll
+        for (int j = 0; j < V; ++j) e[j] = (int)f0 + j < A.F ? src[(int64_t)j * A.sf] : (T)0;
+        __builtin_memcpy(&v, e, 16);
+      }
+      *(u32x4w*)((T*)A.dst + ((int64_t)b * A.K + k) * A.pitch + f0) = v;
+    }
+}
+
+// K-contiguous rows (sk == 1) transposed through LDS, 64 × 64 elements per workgroup: rows are read along k and written
+// along f in 16-byte chunks. (i8 1000 × 1000 × 1000, one operand each way: 68 → 28 µs with the product.)
+template <int ES>
+__global__ void __launch_bounds__(256) pack_transpose_kernel(const PackArgs A) {
+  using T = typename PackElem<ES>::T;
+  constexpr int V = 16 / ES, CPR = 64 / V;   // chunks per 64 elements
+  constexpr int P = 64 * ES + 16;            // LDS row pitch in bytes
+  __shared__ __attribute__((aligned(16))) char tile[64 * P];
+  const int k0 = blockIdx.x * 64;
+  const int fblocks = (A.F + 63) / 64;
+  for (int64_t w = blockIdx.y; w < (int64_t)fblocks * A.batch; w += gridDim.y) {
+    const int b = (int)(w / fblocks), f0 = (int)(w % fblocks) * 64;
+    const T* src = (const T*)A.src + (int64_t)b * A.sb;
+    for (int i = threadIdx.x; i < 64 * CPR; i += 256) {
+      const int f = i / CPR, k = (i % CPR) * V;
+      const T* p = src + (int64_t)(f0 + f) * A.sf + k0 + k;
+      u32x4w v = u32x4w{0, 0, 0, 0};
+      if (f0 + f < A.F) {
+        if (k0 + k + V <= A.K) {
+          v = load_unaligned16((const char*)p);
+        } else {
+          T e[V];
+#pragma unroll
+          for (int j = 0; j < V; ++j) e[j] = k0 + k + j < A.K ? p[j] : (T)0;
+          __builtin_memcpy(&v, e, 16);
+        }
+      }
+      *(u32x4w*)(tile + f * P + k * ES) = v;
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < 64 * CPR; i += 256) {
+      const int k = i / CPR, f = (i % CPR) * V;
+      T e[V];
+#pragma unroll
+      for (int j = 0; j < V; ++j) e[j] = *(const T*)(tile + (f + j) * P + k * ES);
+      u32x4w v;
+      __builtin_memcpy(&v, e, 16);
+      if (k0 + k < A.K && f0 + f < A.pitch) *(u32x4w*)((T*)A.dst + ((int64_t)b * A.K + k0 + k) * A.pitch + f0 + f) = v;
+    }
+    __syncthreads();  // the next block reuses the tile
+  }
+}
+
+template <int ES>
+void launch_pack_es(const PackArgs& a, hipStream_t stream, hipEvent_t done) {
+  if (a.sk == 1 && a.sf != 1 && a.K > 1) {
+    const int64_t blocks = ((int64_t)a.F + 63) / 64 * a.batch;
+    const dim3 grid((unsigned)((a.K + 63) / 64), (unsigned)std::min<int64_t>(blocks, 65535));
+    launch_k(done, pack_transpose_kernel<ES>, grid, dim3(256), 0, stream, a);
+  } else {
+    const int64_t chunks = (int64_t)a.K * (a.pitch * ES / 16);
+    if (chunks > INT32_MAX) fail(PJRT_Error_Code_UNIMPLEMENTED, "dot operand too large to copy");
+    const dim3 grid((unsigned)std::min<int64_t>((chunks + 255) / 256, 65536), (unsigned)std::min(a.batch, 65535));
+    launch_k(done, pack_rows_kernel<ES>, grid, dim3(256), 0, stream, a);
+  }
+}
+
+}  // namespace
+
+void launch_pack(const PackArgs& a, hipStream_t stream, hipEvent_t done) {
+  if (a.batch < 0 || a.K < 0 || a.F < 0 || a.pitch < a.F || a.pitch % 16 || ((uintptr_t)a.dst & 15))
+    fail(PJRT_Error_Code_INTERNAL, "dot operand copy: arguments");
+  if (a.batch == 0 || a.K == 0 || a.F == 0) return record_done(done, stream);
+  switch (a.elem_bytes) {
+    case 1: launch_pack_es<1>(a, stream, done); break;
+    case 2: launch_pack_es<2>(a, stream, done); break;
+    case 4: launch_pack_es<4>(a, stream, done); break;
+    default: fail(PJRT_Error_Code_INTERNAL, "dot operand copy: element size " + std::to_string(a.elem_bytes));
+  }
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) fail(PJRT_Error_Code_INTERNAL, std::string("dot operand copy failed: ") + hipGetErrorString(e));
 }
 
 }  // namespace ryft

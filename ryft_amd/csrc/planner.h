@@ -17,7 +17,7 @@ struct Slot {
 };
 
 struct Step {
-  enum Kind { ELEMENTWISE, REDUCE, GEMM, ATTENTION, COPY, ROW, WINDOW, GATHER, REDUCE_BODY, SCATTER } kind;
+  enum Kind { ELEMENTWISE, REDUCE, GEMM, ATTENTION, COPY, ROW, WINDOW, GATHER, REDUCE_BODY, SCATTER, PACK } kind;
   std::string name;  // kernel family, for profiling ("gemm_bf16_mfma", "attention_fwd", ...)
   EwProgram ew;
   ReduceArgs red;
@@ -28,6 +28,7 @@ struct Step {
   GatherArgs gat;
   ScatterArgs sca;
   ReduceBodyArgs rbody;
+  PackArgs pack;
   struct { int64_t bytes; int64_t src_offset; } copy;  // src_offset: bytes into the source slot
   // Pointer fields inside the args block that refer to slots: (byte offset of the pointer field, slot). The
   // field's initial value is a byte offset into the slot's buffer.
@@ -45,6 +46,7 @@ struct Step {
       case GATHER: return &gat;
       case SCATTER: return &sca;
       case REDUCE_BODY: return &rbody;
+      case PACK: return &pack;
       default: return nullptr;
     }
   }

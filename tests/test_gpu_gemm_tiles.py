@@ -47,6 +47,26 @@ def test_gemm_tiles(gpu_client, case):
     print(f"[tiles] {name} {plan.splitlines()[-1].split('tile=')[1].split(' flops')[0]} error {err:.2e}", flush=True)
 
 
+# operands whose rows the loads cannot read, copied into padded rows first: the copy keeps the layout of a
+# free-contiguous operand and transposes a K-contiguous one, in blocks of 64 × 64 and vectors of 16 bytes
+PACKED = [dot("bf16_both_transposed", (67, 1001), (129, 1001), "bf16", "f32", [1], [1], seed=51),
+          dot("bf16_lhs_transposed_rhs_rows", (3, 65, 63), (3, 63, 71), "bf16", "f32", [2], [1], [0], [0], seed=52),
+          dot("bf16_free_contiguous", (130, 67), (130, 201), "bf16", "f32", [0], [0], seed=53),
+          dot("i8_odd", (17, 333), (333, 31), "i8", "i32", [1], [0], seed=54),
+          dot("i8_odd_transposed", (65, 130), (129, 130), "i8", "i32", [1], [1], seed=55),
+          dot("f32_odd", (65, 131), (131, 67), "f32", "f32", [1], [0], seed=56),
+          dot("fp8_odd", (33, 77), (77, 19), "f8E4M3FN", "f32", [1], [0], seed=57),
+          dot("bf16_f8_odd", (5, 72), (72, 999), "bf16", "f32", [1], [0], rhs_dt="f8E4M3FN", seed=58)]
+
+
+@pytest.mark.parametrize("case", PACKED, ids=[c[0] for c in PACKED])
+def test_unaligned_operands(gpu_client, case):
+    name, prog, ins = case
+    outs, exe = run_pjrt(gpu_client, prog, ins)
+    assert "dot_operand_copy" in exe.describe_plan() and "generic" not in exe.describe_plan()
+    check(outs[0], oracle_outputs(prog, ins)[0], BF16, name)
+
+
 @pytest.mark.parametrize("kw", [dict(m=1, d=1024, f=2048), dict(m=16, d=2048, f=1040), dict(m=33, d=1040, f=2048),
                                 dict(m=77, d=1280, f=2048), dict(m=130, d=512, f=528)])
 def test_swiglu_of_few_rows(gpu_client, kw):
