@@ -228,7 +228,7 @@ struct GemmArgs {
   // workgroups of range s write their raw f32 / i32 accumulators to ws[s][acc][batch][M][N] (acc: 0, and 1 for the
   // second dot of a dual GEMM), and a reduction kernel sums the ranges in order and applies the epilogue.
   int32_t splits;
-  int32_t pad_splits;
+  int32_t family;  // MFMA kernels: 1 full tiles, 2 edge tiles (set by gemm_plan_family); 0: full tiles where they fit
   void* ws;
   // split-K with per-output-tile arrival counters (zero between launches; the finishing range sets its tile's back
   // to zero): the K range that completes a tile last sums the ranges' partial sums and applies the epilogue inside

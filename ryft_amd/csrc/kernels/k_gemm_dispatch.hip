@@ -208,27 +208,30 @@ static bool edge_splittable(const GemmArgs& g, const Choice& c, int splits) {
          (int64_t)(splits - 1) * per < kt;
 }
 
-// Microseconds of one k-tile (128 bytes of k per row; 64 for f32) of an edge tile: `alone`, of a workgroup with a CU to
+// Microseconds of one k-tile (128 bytes of k per row; 64 for f32) of a tile: `alone`, of a workgroup with a CU to
 // itself, and `shared`, per workgroup of a busy CU. Measured at (M, K, N) = (1, 4096, 4096), (16, 4096, 14336),
-// (64, 4096, 4096), (300, 4096, 8192), (1000, 1000, 1000), (2000, 3000, 4000) and others, every tile and split of each:
-// small tiles move more operand bytes per product (a 64×64 tile's k-tile takes 0.27 µs whether the CU runs one or eight
-// of them: it is the L2-to-LDS rate, about 60 GB/s per CU) but there are more of them to fill the chip with.
+// (64, 4096, 4096), (300, 4096, 8192), (512, 4096, 4096), (1000, 1000, 1000), (2000, 3000, 4000) and others, every tile
+// and split of each: small tiles move more operand bytes per product (a 64×64 tile's k-tile takes 0.2-0.27 µs whether
+// the CU runs one or eight of them: it is the L2-to-LDS rate, about 60 GB/s per CU) but there are more of them to fill
+// the chip with, and their four LDS stages hide the load latency that two stages of a 128×128 tile alone on a CU do not.
 struct TileTime {
   int kind, bm, bn, dual;
   double alone, shared;
 };
 static constexpr TileTime kTileTimes[] = {
-    {MMA_BF16, 256, 256, 0, 1.4, 1.95},    {MMA_BF16, 128, 128, 0, 0.77, 0.56},   {MMA_BF16, 64, 64, 0, 0.27, 0.27},
-    {MMA_BF16, 32, 128, 0, 0.29, 0.275},   {MMA_F16, 128, 128, 0, 0.77, 0.56},    {MMA_I8, 256, 256, 0, 1.4, 2.0},
-    {MMA_I8, 128, 128, 0, 0.9, 0.7},       {MMA_I8, 64, 128, 0, 0.45, 0.42},      {MMA_I8, 32, 128, 0, 0.3, 0.27},
-    {MMA_FP8, 128, 128, 0, 0.9, 0.7},      {MMA_FP8, 128, 128, 1, 1.4, 1.0},      {MMA_F32, 64, 64, 0, 0.45, 0.38},
-    {MMA_BF16_F8, 128, 128, 0, 0.9, 0.46}, {MMA_BF16_F8, 64, 128, 0, 0.38, 0.24}, {MMA_BF16_F8, 32, 128, 0, 0.28, 0.18},
-    {MMA_BF16_F8, 128, 128, 1, 1.3, 1.0},  {MMA_BF16_F8, 64, 128, 1, 0.66, 0.65}, {MMA_BF16_F8, 32, 128, 1, 0.6, 0.34}};
+    {MMA_BF16, 256, 256, 0, 1.4, 1.95},    {MMA_BF16, 256, 128, 0, 0.9, 0.9},     {MMA_BF16, 128, 128, 0, 0.77, 0.56},
+    {MMA_BF16, 64, 64, 0, 0.27, 0.22},     {MMA_BF16, 32, 128, 0, 0.29, 0.26},    {MMA_F16, 128, 128, 0, 0.77, 0.56},
+    {MMA_I8, 256, 256, 0, 1.4, 2.0},       {MMA_I8, 128, 128, 0, 0.9, 0.7},       {MMA_I8, 64, 128, 0, 0.45, 0.42},
+    {MMA_I8, 32, 128, 0, 0.3, 0.27},       {MMA_FP8, 128, 128, 0, 0.9, 0.7},      {MMA_FP8, 64, 128, 0, 0.6, 0.45},
+    {MMA_FP8, 128, 128, 1, 1.4, 1.0},      {MMA_F32, 64, 64, 0, 0.45, 0.38},      {MMA_BF16_F8, 256, 256, 0, 1.6, 2.0},
+    {MMA_BF16_F8, 128, 256, 0, 1.25, 1.2}, {MMA_BF16_F8, 128, 128, 0, 0.9, 0.62}, {MMA_BF16_F8, 64, 128, 0, 0.38, 0.29},
+    {MMA_BF16_F8, 32, 128, 0, 0.28, 0.25}, {MMA_BF16_F8, 256, 128, 1, 1.33, 1.6},  {MMA_BF16_F8, 128, 128, 1, 1.3, 1.0},
+    {MMA_BF16_F8, 64, 128, 1, 0.66, 0.65}, {MMA_BF16_F8, 32, 128, 1, 0.6, 0.45}};
 
-// Estimated microseconds of an edge tile over `splits` K ranges: the k-tiles of the busiest CU's workgroups, and for a
+// Estimated microseconds of a tile over `splits` K ranges: the k-tiles of the busiest CU's workgroups, and for a
 // split the arrival and finish in-kernel (partial sums up to 8 MiB) or the reduction launch, both growing with the
 // partial sums' traffic.
-static double edge_cost(const GemmArgs& g, int kind, const Choice& c, int splits) {
+static double tile_cost(const GemmArgs& g, int kind, const Choice& c, int splits) {
   const TileTime* t = nullptr;
   for (const TileTime& x : kTileTimes)
     if (x.kind == kind && x.bm == c.bm && x.bn == c.bn && x.dual == (g.dual ? 1 : 0)) t = &x;
@@ -239,7 +242,7 @@ static double edge_cost(const GemmArgs& g, int kind, const Choice& c, int splits
   double us = 3.0 + per * each;
   if (splits > 1) {
     const double mb = (double)splits * (g.dual ? 2 : 1) * g.batch * g.M * g.N * 4.0 / (1 << 20);
-    us += mb <= 8.0 ? 3.0 + 0.5 * mb : 5.5 + 0.55 * mb;
+    us += mb <= 8.0 ? 3.0 + 0.5 * mb : 8.0 + 0.3 * mb;
   }
   return us;
 }
@@ -260,7 +263,7 @@ static bool pick_edge_tile(const GemmArgs& g, int kind, bool ar, bool br, Choice
   const int splits = std::max(1, (int)g.splits);
   for (int i = 0; i < n; ++i) {
     if (g.splits > 1 && !edge_splittable(g, t[i], g.splits)) continue;
-    if (best < 0 || edge_cost(g, kind, t[i], splits) < edge_cost(g, kind, t[best], splits)) best = i;
+    if (best < 0 || tile_cost(g, kind, t[i], splits) < tile_cost(g, kind, t[best], splits)) best = i;
   }
   if (best < 0) return false;
   *c = t[best];
@@ -284,11 +287,13 @@ static bool pick_mfma(const GemmArgs& g, Choice* c) {
   const int bes = kind == MMA_BF16_F8 ? 1 : es;  // B's element size in HBM
   int ar = 0, br = 0;
   if (layout_gaps(g, kind, &ar, &br)) return false;
-  bool ok = pick_full(g, kind, ar, br, c);
-  // (shapes that run full tiles are split over full tiles or not at all)
-  GemmArgs whole = g;
-  whole.splits = 1;
-  if (!ok && !(g.splits > 1 && pick_full(whole, kind, ar, br, c))) ok = pick_edge_tile(g, kind, ar, br, c);
+  bool ok = g.family != 2 && pick_full(g, kind, ar, br, c);
+  if (!ok && g.family != 1) {
+    // (shapes that run full tiles are split over full tiles or not at all)
+    GemmArgs whole = g;
+    whole.splits = 1;
+    if (g.family == 2 || !(g.splits > 1 && pick_full(whole, kind, ar, br, c))) ok = pick_edge_tile(g, kind, ar, br, c);
+  }
   if (ok && c->edge) {
     // the edge kernels zero k positions past K a load at a time: K must end on a load boundary of each
     // K-contiguous operand (16-byte vectors; 8-byte pieces for a widened f8 B)
@@ -340,11 +345,11 @@ int gemm_plan_splits(const GemmArgs& a) {
   if (c.edge) {
     int best = 1;
     const int kind = mma_kind(g);
-    double cost = edge_cost(g, kind, c, 1);
+    double cost = tile_cost(g, kind, c, 1);
     for (int s = 2; s <= 16; s *= 2) {
       g.splits = s;
       if (!pick_mfma(g, &c)) continue;
-      const double t = edge_cost(g, kind, c, s);
+      const double t = tile_cost(g, kind, c, s);
       if (t < cost) best = s, cost = t;
     }
     return best;
@@ -370,6 +375,29 @@ int gemm_plan_splits(const GemmArgs& a) {
   if (best < 2 || (!small_tile && tiles_s * best <= tiles)) return 1;
   g.splits = best;
   return pick_mfma(g, &c) ? best : 1;
+}
+
+int gemm_plan_family(const GemmArgs& a) {
+  // Full tiles where they fit, unless the edge family (smaller tiles, deeper pipelines, more ways to split) is estimated
+  // to save a fifth of the time and 6 µs, the estimates' own error. Both sides measured: bf16 1024³ 19.6 µs in full
+  // tiles over 4 K ranges, 7.5 in 64×64 tiles; 512 × 4096 × 4096 36 and 28; i8 512 × 4096 × 4096 32.5 and 21.5; f8
+  // weights [11648, 2304] for 128 rows 128 and 24, [14336, 4096] for 1024 rows 211 and 136; for 512 rows (82 and 83)
+  // and for 2048³ (29 and 31) the full tiles stay.
+  GemmArgs g = a;
+  g.splits = 1;
+  const int kind = mma_kind(g);
+  double cost[3] = {0, 0, 0};
+  for (int f = 1; f <= 2; ++f) {
+    Choice c;
+    g.family = f;
+    g.splits = 1;
+    if (!pick_mfma(g, &c)) return f == 1 ? 2 : 1;
+    const int s = gemm_plan_splits(g);
+    g.splits = s;
+    if (s > 1 && !pick_mfma(g, &c)) return 1;
+    cost[f] = tile_cost(g, kind, c, s);
+  }
+  return cost[2] < 0.8 * cost[1] && cost[2] < cost[1] - 6.0 ? 2 : 1;
 }
 
 void launch_gemm(const GemmArgs& g, hipStream_t stream, hipEvent_t done) {

@@ -31,6 +31,8 @@ int gemm_mfma_layout_gaps(const GemmArgs& a);
 const char* gemm_kernel_name(const GemmArgs& a);
 // Whether launch_gemm() runs these arguments on an edge kernel (its name stands for the family), and on which tile.
 bool gemm_edge_tile(const GemmArgs& a, int* bm, int* bn);
+// The tile family (GemmArgs::family) launch_gemm should run these unsplit arguments in.
+int gemm_plan_family(const GemmArgs& a);
 // Number of K ranges launch_gemm splits these arguments into when given a workspace of
 // splits × (dual ? 2 : 1) × batch × M × N 4-byte accumulators (1: no split).
 int gemm_plan_splits(const GemmArgs& a);

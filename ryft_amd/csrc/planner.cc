@@ -1785,6 +1785,7 @@ void Planner::emit_dot(const std::vector<int>& dots_in, int target, int root) {
     G.epilogue = EPI_STORE;
     st.patches.push_back({offsetof(GemmArgs, out_ptr), out});
     st.bytes += (double)d.type.bytes();
+    G.family = gemm_plan_family(G);
     st.name = gemm_kernel_name(G);
     plan_split_k(st);
     plan_.steps.push_back(std::move(st));
@@ -1852,6 +1853,7 @@ void Planner::emit_dot(const std::vector<int>& dots_in, int target, int root) {
       return;
     }
   }
+  G.family = gemm_plan_family(G);
   st.name = gemm_kernel_name(G);
   plan_split_k(st);
   plan_.steps.push_back(std::move(st));

@@ -20,7 +20,7 @@ CASES = [
     (dot("bf16_64_tiles", (1000, 1000), (1000, 1000), "bf16", "f32", [1], [0], seed=33), "64x64", False),
     (dot("bf16_k_contiguous_both", (65, 2056), (1031, 2056), "bf16", "f32", [1], [1], seed=34), None, False),
     (dot("bf16_m_contiguous_tail", (1001, 136), (1001, 264), "bf16", "f32", [0], [0], seed=35), None, True),
-    (dot("bf16_128_tiles", (2000, 520), (520, 2056), "bf16", "f32", [1], [0], seed=36), "128x128", False),
+    (dot("bf16_128_tiles", (2000, 520), (520, 4088), "bf16", "f32", [1], [0], seed=36), "128x128", False),
     (dot("bf16_256_tiles", (136, 4088), (136, 4088), "bf16", "f32", [0], [0], seed=37), "256x256", False),
     (dot("bf16_256_tiles_k_contiguous_b", (72, 4096), (4088, 72), "bf16", "f32", [0], [1], seed=38), "256x256", False),
     (dot("i8_one_row", (1, 4096), (4096, 2064), "i8", "i32", [1], [0], seed=39), "32x128", True),
