@@ -366,10 +366,58 @@ class _Owned:
         return obj
 
 
+# What belongs to a client — buffers, executables and their completion events — is tracked by its handle and destroyed
+# before the client is. The wrappers refer to their client, but that keeps the order only while they die by reference
+# count: the garbage collector finalizes the objects of an unreachable cycle (a caught exception's frames, say) in any
+# order, a client before its buffers among them, and a buffer destroyed after its client would return its memory to an
+# allocator that is gone. Each object is destroyed by whoever takes its handle out of its one-element claim list — the
+# wrapper's finalizer, its client's or the exit hook; taking it is atomic, and a claim is never another object's, as a
+# handle the plugin has reused could be. (An entry is also cheaper than a weak reference to each wrapper.)
+_LIVE_HANDLES: Dict[int, Tuple["Api", str, int, List[int]]] = {}  # id(claim) → api, destroy function, client, claim
+
+
+class _OwnedHandle:
+    _destroy = ""
+
+    def _own(self, api: "Api", handle: int, client: int):
+        self.handle = handle
+        self._claim = claim = [handle]
+        _LIVE_HANDLES[id(claim)] = (api, self._destroy, client, claim)
+
+    def __del__(self):
+        try:
+            handle = self._claim.pop()
+        except (AttributeError, IndexError):  # never owned, or destroyed with its client
+            return
+        try:
+            self.handle = None
+            api, name = _LIVE_HANDLES.pop(id(self._claim))[:2]
+            api.destroy(name, handle)
+        except Exception:
+            pass
+
+
+def _destroy_handles(client: Optional[int] = None):
+    """Destroys the tracked objects of one client (None: of every client)."""
+    for key, (api, name, owner, claim) in list(_LIVE_HANDLES.items()):
+        if client is not None and owner != client:
+            continue
+        try:
+            handle = claim.pop()
+        except IndexError:
+            continue
+        _LIVE_HANDLES.pop(key, None)
+        try:
+            api.destroy(name, handle)
+        except Exception:
+            pass
+
+
 @atexit.register
 def _destroy_live_objects():
     for obj in sorted(list(_LIVE.values()), key=lambda o: o._exit_order):
         obj.__del__()
+    _destroy_handles()
 
 
 class LayoutsExtension:
@@ -522,6 +570,13 @@ class Api:
         if err is not None:
             raise err
         return args
+
+    def destroy(self, name: str, handle: int):
+        """The table's destroy function `name` on `handle` (args: struct size, extension, handle)."""
+        args = A[name]
+        err = self.fn(name)(C.byref(args(C.sizeof(args), None, handle)))
+        if err:
+            raise self.error(err)
 
     def extension(self, ext_type: int):
         p = C.c_void_p.from_address(self.handle + 8).value
@@ -735,14 +790,17 @@ class Device:
 
 
 # ----------------------------------------------------------------------------------------------- events
-class Event(_Owned):
+class Event(_OwnedHandle):
     """PJRT_Event wrapper (events.rs); `await_` blocks, `on_ready` registers a callback."""
 
-    def __init__(self, api: Api, handle: int, value=None):
+    def __init__(self, api: Api, handle: int, value=None, client: int = 0):
         if not handle:
             raise PjrtError(ErrorCode.INVALID_ARGUMENT, "the provided PJRT event handle is a null pointer")
-        self.api, self.handle, self._value = api, handle, value
+        self.api, self._value = api, value
         self._callbacks = []
+        self._own(api, handle, client)
+
+    _destroy = "PJRT_Event_Destroy"
 
     def is_ready(self) -> bool:
         return self.api.call("PJRT_Event_IsReady", event=self.handle).is_ready
@@ -758,21 +816,19 @@ class Event(_Owned):
         self._callbacks.append(c)  # kept alive with the event
         self.api.call("PJRT_Event_OnReady", event=self.handle, callback=c, user_arg=None)
 
-    def __del__(self):
-        try:
-            if self.handle:
-                self.api.call("PJRT_Event_Destroy", event=self.handle)
-                self.handle = None
-        except Exception:
-            pass
-
 
 # ----------------------------------------------------------------------------------------------- buffers
-class Buffer(_Owned):
+_UNSAFE_POINTER_ARGS = A["PJRT_Buffer_UnsafePointer"]
+
+
+class Buffer(_OwnedHandle):
+    _destroy = "PJRT_Buffer_Destroy"
+
     def __init__(self, client: "Client", handle: int):
         if not handle:
             raise PjrtError(ErrorCode.INVALID_ARGUMENT, "the provided PJRT buffer handle is a null pointer")
-        self.client, self.handle = client, handle
+        self.client = client
+        self._own(client.api, handle, client.handle)
 
     @property
     def api(self) -> Api:
@@ -817,7 +873,11 @@ class Buffer(_Owned):
 
     def unsafe_pointer(self) -> int:
         """Buffer::unsafe_pointer (buffers.rs:1500-1505): the device address of the buffer's bytes."""
-        return int(self.api.call("PJRT_Buffer_UnsafePointer", buffer=self.handle).buffer_pointer)
+        args = _UNSAFE_POINTER_ARGS(C.sizeof(_UNSAFE_POINTER_ARGS), None, self.handle, 0)
+        err = self.client.api.fn("PJRT_Buffer_UnsafePointer")(C.byref(args))
+        if err:
+            raise self.api.error(err)
+        return args.buffer_pointer
 
     def copy_to_host(self) -> Event:
         """ToHostBuffer twice: size query with dst=null, then the copy (buffers.rs:1237-1266)."""
@@ -858,14 +918,6 @@ class Buffer(_Owned):
                               dst_size=size)
             Event(self.api, a.event).await_()
         return out
-
-    def __del__(self):
-        try:
-            if self.handle:
-                self.api.call("PJRT_Buffer_Destroy", buffer=self.handle)
-                self.handle = None
-        except Exception:
-            pass
 
 
 # ----------------------------------------------------------------------------------------------- programs
@@ -997,9 +1049,12 @@ class ExecutionContext(_Owned):
             pass
 
 
-class Executable(_Owned):
-    def __init__(self, api: Api, handle: int):
-        self.api, self.handle = api, handle
+class Executable(_OwnedHandle, _Owned):
+    _destroy = "PJRT_Executable_Destroy"
+
+    def __init__(self, api: Api, handle: int, client: int = 0):
+        self.api = api
+        self._own(api, handle, client)
 
     def name(self) -> str:
         a = self.api.call("PJRT_Executable_Name", executable=self.handle)
@@ -1072,14 +1127,6 @@ class Executable(_Owned):
         a = self.api.call("PJRT_Executable_OutputMemoryKinds", executable=self.handle)
         return [_str(a.memory_kinds[i], a.memory_kind_sizes[i]) for i in range(a.num_outputs)]
 
-    def __del__(self):
-        try:
-            if self.handle:
-                self.api.call("PJRT_Executable_Destroy", executable=self.handle)
-                self.handle = None
-        except Exception:
-            pass
-
 
 @dataclass
 class ExecutionInput:
@@ -1093,11 +1140,18 @@ class ExecutionDeviceOutputs:
     done: Event
 
 
-class LoadedExecutable(_Owned):
+_BUFFER_ONLY = frozenset([Buffer])
+
+
+class LoadedExecutable(_OwnedHandle, _Owned):
+    _destroy = "PJRT_LoadedExecutable_Destroy"
+
     def __init__(self, client: "Client", handle: int):
         if not handle:
             raise PjrtError(ErrorCode.INVALID_ARGUMENT, "the provided PJRT loaded executable handle is a null pointer")
-        self.client, self.handle = client, handle
+        self.client = client
+        self._counts, self._local = None, threading.local()
+        self._own(client.api, handle, client.handle)
 
     @property
     def api(self) -> Api:
@@ -1109,7 +1163,7 @@ class LoadedExecutable(_Owned):
 
     def executable(self) -> Executable:
         a = self.api.call("PJRT_LoadedExecutable_GetExecutable", loaded_executable=self.handle)
-        return Executable(self.api, a.executable)
+        return Executable(self.api, a.executable, self.client.handle)
 
     def device_assignment(self) -> DeviceAssignment:
         """LoadedExecutable::device_assignment (programs.rs:704-736; decoding as devices.rs:674-688)."""
@@ -1120,20 +1174,18 @@ class LoadedExecutable(_Owned):
 
     def execute(self, inputs: Sequence[Sequence], launch_id: int = 0) -> List[ExecutionDeviceOutputs]:
         """LoadedExecutable::execute (programs.rs:769-963): one input list per addressable device."""
-        counts = self.__dict__.get("_counts")
+        counts = self._counts
         if counts is None:  # fixed for a loaded executable: queried once, not on every execution
             counts = self._counts = (len(self.addressable_devices()), self.executable().output_count())
         device_count, output_count = counts
         # Repeated executions on the same plain (non-donated) buffers of one device reuse a prepared argument block
         # (per thread: the call releases the GIL, and its output arrays are written during it).
-        if device_count == 1 and len(inputs) == 1 and all(type(x) is Buffer for x in inputs[0]):
-            local = self.__dict__.get("_local")
-            if local is None:
-                local = self._local = threading.local()
-            prepared = getattr(local, "prepared", None)
-            if prepared is None:
-                prepared = local.prepared = {}
-            key = (tuple(x.handle for x in inputs[0]), launch_id)
+        if device_count == 1 and len(inputs) == 1 and _BUFFER_ONLY.issuperset(map(type, inputs[0])):
+            try:
+                prepared = self._local.prepared
+            except AttributeError:
+                prepared = self._local.prepared = {}
+            key = (launch_id, *[x.handle for x in inputs[0]])
             prep = prepared.get(key)
             if prep is None:
                 if len(prepared) >= 32:
@@ -1141,10 +1193,11 @@ class LoadedExecutable(_Owned):
                 prep = prepared[key] = self._prepare(inputs[0], launch_id, output_count)
             args, ref, outs, events, fn = prep
             err = fn(ref)
+            client = self.client
             if err:
-                raise self.api.error(err)
-            return [ExecutionDeviceOutputs([Buffer(self.client, outs[o]) for o in range(output_count)],
-                                           Event(self.api, events[0]))]
+                raise client.api.error(err)
+            return [ExecutionDeviceOutputs([Buffer(client, outs[o]) for o in range(output_count)],
+                                           Event(client.api, events[0], None, client.handle))]
         if len(inputs) != device_count:
             raise PjrtError(ErrorCode.INVALID_ARGUMENT,
                             f"expected inputs for {device_count} device(s) but got inputs for {len(inputs)} device(s)")
@@ -1215,14 +1268,6 @@ class LoadedExecutable(_Owned):
         if err:
             raise err
         return _str(p.value, n.value)
-
-    def __del__(self):
-        try:
-            if self.handle:
-                self.api.call("PJRT_LoadedExecutable_Destroy", executable=self.handle)
-                self.handle = None
-        except Exception:
-            pass
 
 
 # ----------------------------------------------------------------------------------------------- client
@@ -1419,6 +1464,7 @@ class Client(_Owned):
     def __del__(self):
         try:
             if self.handle:
+                _destroy_handles(self.handle)
                 self.api.call("PJRT_Client_Destroy", client=self.handle)
                 self.handle = None
         except Exception:

@@ -702,3 +702,30 @@ def test_malformed_aliasing_is_invalid_argument(compile_client, name):
     with pytest.raises(pjrt.PjrtError) as e:
         compile_client.compile(pjrt.Program.mlir(program))
     assert e.value.code == pjrt.ErrorCode.INVALID_ARGUMENT and fragment in str(e.value), str(e.value)
+
+
+def test_client_in_a_reference_cycle_outlives_what_it_owns(plugin):
+    """The garbage collector may finalize the objects of an unreachable cycle in any order: a client collected together
+    with its executables (a caught exception's frames hold both, for one) is still destroyed after them."""
+    import gc
+
+    client = plugin.client({"compile_only": True})
+    exe = client.compile(pjrt.Program.mlir(ADD_2X1))
+    inner = exe.executable()
+    order = []
+    api = plugin.api()
+    names = ("PJRT_Client_Destroy", "PJRT_LoadedExecutable_Destroy", "PJRT_Executable_Destroy")
+    real = {n: api.fn(n) for n in names}
+    gc.collect()
+    gc.disable()
+    try:
+        for n in names:
+            api._fns[n] = lambda ref, n=n: (order.append(n), real[n](ref))[1]
+        cycle = [client, exe, inner]
+        cycle.append(cycle)
+        del client, exe, inner, cycle
+        gc.collect()
+    finally:
+        api._fns.update(real)
+        gc.enable()
+    assert sorted(order) == sorted(names) and order[-1] == "PJRT_Client_Destroy", order
