@@ -966,6 +966,89 @@ __global__ void __launch_bounds__(VNT) rownorm_block_kernel(const RowArgs A) {
   }
 }
 
+// RMSNorm rows that are no multiple of 8 elements, so that neither their starts nor the weights' vectors line up: thread
+// t of a row's G owns elements t, t + G, ..., eight in flight at a time (loads past the row's end re-read its last
+// element, unused), every access of a wavefront one run of 64 elements. Folded in the order of the interpreted row
+// kernel for such rows (same G, same bits), which it replaces there: interpreting the program element by element was
+// bound by its own instructions, not by memory or latency. The scaling pass reads the row again, from L2.
+// bf16 passes on the host's clock, interpreted → here: 1 × 16383 498 → 13 µs, 170 × 1001 148 → 13, 4000 × 16377
+// 2543 → 76 (3.4 TB/s). What bounds it: few rows the launch and the chain of loads, many rows the 2-byte accesses.
+template <int G>
+__device__ __forceinline__ void load8_strided(const void* p, int64_t base, int64_t i, int64_t last, int dt, float* v) {
+  int64_t at[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) at[e] = base + (i + e * G < last ? i + e * G : last);
+  if (dt == DT_F32) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = ((const float*)p)[at[e]];
+  } else if (dt == DT_BF16) {
+    uint32_t w[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) w[e] = ((const uint16_t*)p)[at[e]];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = __uint_as_float(w[e] << 16);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = (float)((const _Float16*)p)[at[e]];
+  }
+}
+
+template <int G>
+__global__ void __launch_bounds__(VNT) rownorm_ragged_kernel(const RowArgs A) {
+#pragma clang fp contract(off)
+  __shared__ float part[VNT / 64];
+  const RowNormArgs& N = A.norm;
+  constexpr int RB = VNT / G;  // rows per workgroup
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, t = threadIdx.x % G;
+  const int64_t last = A.inner - 1;
+  for (int64_t o = (int64_t)blockIdx.x * RB + threadIdx.x / G; o < A.rows; o += (int64_t)gridDim.x * RB) {
+    const int64_t base = o * A.inner;
+    float acc = 0.0f;
+    for (int64_t i = t; i < A.inner; i += 8 * G) {
+      float v[8];
+      load8_strided<G>(N.x, base, i, last, N.x_dtype, v);
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (i + e * G <= last) acc = acc + v[e] * v[e];
+    }
+    for (int off = 32; off > 0; off >>= 1) acc = acc + __shfl_xor(acc, off, 64);
+    acc = __shfl(acc, 0, 64);
+    if constexpr (G == VNT) {
+      if (lane == 0) part[wave] = acc;
+      __syncthreads();
+      acc = part[0];
+      for (int w = 1; w < VNT / 64; ++w) acc = acc + part[w];
+      __syncthreads();
+    }
+    const float s = rownorm_scale(A, acc);
+    for (int64_t i = t; i < A.inner; i += 8 * G) {
+      float y[8];
+      load8_strided<G>(N.x, base, i, last, N.x_dtype, y);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) y[e] = y[e] * s;
+      if (N.w) {
+        float wv[8];
+        load8_strided<G>(N.w, 0, i, last, N.w_dtype, wv);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) y[e] = y[e] * wv[e];
+      }
+      round8(y, N.mid_round);
+      auto put = [&](int dt) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (i + e * G <= last) store_bits(N.out, base + i + e * G, dt, __float_as_uint(y[e]), true);
+      };
+      switch (N.out_dtype) {
+        case DT_F32: put(DT_F32); break;
+        case DT_BF16: put(DT_BF16); break;
+        case DT_F16: put(DT_F16); break;
+        case DT_F8E4M3FN: put(DT_F8E4M3FN); break;
+        default: put(DT_F8E5M2); break;
+      }
+    }
+  }
+}
+
 // Whether a [rows, inner] row step gives each row one wavefront (else one workgroup), in the interpreted row kernel
 // and in the RMSNorm kernels alike, so both fold a row's sums in the same order: short rows always; rows of up to
 // ROW_WAVE_CHUNKS 8-element vectors when there are enough of them to keep every compute unit's waves busy (with few
@@ -989,14 +1072,18 @@ static int rownorm_rows_per_cu() {
   return n;
 }
 
-static bool rownorm_launchable(const RowArgs& a) {
-  const RowNormArgs& n = a.norm;
+static bool rownorm_types(const RowNormArgs& n) {
   auto float_ok = [](int dt) { return dt == DT_F32 || dt == DT_BF16 || dt == DT_F16; };
-  auto aligned = [](const void* p) { return ((uintptr_t)p & 15u) == 0; };
-  return a.inner % 8 == 0 && float_ok(n.x_dtype) && (!n.w || float_ok(n.w_dtype)) && aligned(n.x) &&
-         (!n.w || aligned(n.w)) && ((uintptr_t)n.out % (uintptr_t)(8 * elem_size(n.out_dtype))) == 0 &&
+  return float_ok(n.x_dtype) && (!n.w || float_ok(n.w_dtype)) &&
          (n.out_dtype == DT_F32 || n.out_dtype == DT_BF16 || n.out_dtype == DT_F16 || n.out_dtype == DT_F8E4M3FN ||
           n.out_dtype == DT_F8E5M2);
+}
+
+static bool rownorm_launchable(const RowArgs& a) {
+  const RowNormArgs& n = a.norm;
+  auto aligned = [](const void* p) { return ((uintptr_t)p & 15u) == 0; };
+  return a.inner % 8 == 0 && rownorm_types(n) && aligned(n.x) && (!n.w || aligned(n.w)) &&
+         ((uintptr_t)n.out % (uintptr_t)(8 * elem_size(n.out_dtype))) == 0;
 }
 
 template <int G, int V>
@@ -1069,6 +1156,17 @@ void launch_row(const RowArgs& a, hipStream_t stream, hipEvent_t done) {
       else if (per_thread <= 4) launch_k(done, rownorm_block_kernel<4>, grid, block, 0, stream, a);
       else launch_k(done, rownorm_block_kernel<0>, grid, block, 0, stream, a);
     }
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) fail(PJRT_Error_Code_INTERNAL, std::string("row-norm launch failed: ") + hipGetErrorString(e));
+    return;
+  }
+  if (a.fast == ROW_FAST_NORM && a.inner % 8 != 0 && rownorm_types(a.norm)) {
+    // rows that are no multiple of 8: a workgroup or a wavefront per row as the interpreted kernel below, which takes
+    // 40 × 4097 in 152 µs against 13 here, 600 × 300 in 58 against 13 (whole vectors at a misaligned start stay there)
+    const bool wide = a.inner >= 4 * VNT;
+    const int64_t blocks = std::min<int64_t>(wide ? a.rows : (a.rows + 3) / 4, 256 * 16);
+    if (wide) launch_k(done, rownorm_ragged_kernel<VNT>, dim3((unsigned)blocks), dim3(VNT), 0, stream, a);
+    else launch_k(done, rownorm_ragged_kernel<64>, dim3((unsigned)blocks), dim3(VNT), 0, stream, a);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) fail(PJRT_Error_Code_INTERNAL, std::string("row-norm launch failed: ") + hipGetErrorString(e));
     return;

@@ -77,6 +77,25 @@ def test_rmsnorm_fast_path_matches_interpreter(gpu_client, interp_client, shape,
     check(fast[0], want, 1e-5 if dt == "f32" else (3e-2 if quant else 1e-2), f"rmsnorm{shape}")
 
 
+@pytest.mark.parametrize("shape,dt,quant", [((1, 33), "f32", None), ((5, 63), "bf16", None), ((7, 513), "f32", None),
+                                            ((4099, 1023), "bf16", "f8E4M3FN"), ((3, 1025), "bf16", None),
+                                            ((5, 2047), "f32", None), ((4097, 2049), "bf16", "f8E4M3FN"),
+                                            ((2, 16383), "bf16", None), ((2, 3, 4100), "bf16", "f8E4M3FN")])
+def test_rmsnorm_ragged_rows_match_interpreter(gpu_client, interp_client, shape, dt, quant):
+    # rows that are no multiple of 8: a wavefront each up to 1023 elements, a workgroup each above; around one and
+    # several batches of eight elements per thread, and more rows than workgroups. Identical bits, as above.
+    d = shape[-1]
+    mk = _f32 if dt == "f32" else _bf16
+    ins = [mk(53, shape), mk(54, (d,), 1.0, 0.02)]
+    prog = row_programs.rmsnorm(shape, dt, quant=quant)
+    fast, exe = run_pjrt(gpu_client, prog, ins)
+    assert exe.describe_plan().split()[1] == "row_norm"
+    slow, _ = run_pjrt(interp_client, prog, ins)
+    assert np.array_equal(fast[0], slow[0]), f"{np.count_nonzero(fast[0] != slow[0])} differing elements"
+    # the bounds of the whole-vector rows above: f32 sums in another order, one bf16 rounding, one f8 step
+    check(fast[0], oracle_outputs(prog, ins)[0], 1e-5 if dt == "f32" else (3e-2 if quant else 1e-2), f"rmsnorm{shape}")
+
+
 @pytest.mark.parametrize("weights", ["finite", "special"])
 def test_rmsnorm_f8_rows_with_special_values(gpu_client, interp_client, weights):
     # many bf16 rows (a wavefront takes several): rows holding +NaN, -NaN, ±inf, an all-zero row (s = rsqrt(eps)),
