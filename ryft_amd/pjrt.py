@@ -366,23 +366,28 @@ class _Owned:
         return obj
 
 
-# What belongs to a client — buffers, executables and their completion events — is tracked by its handle and destroyed
-# before the client is. The wrappers refer to their client, but that keeps the order only while they die by reference
-# count: the garbage collector finalizes the objects of an unreachable cycle (a caught exception's frames, say) in any
-# order, a client before its buffers among them, and a buffer destroyed after its client would return its memory to an
-# allocator that is gone. Each object is destroyed by whoever takes its handle out of its one-element claim list — the
-# wrapper's finalizer, its client's or the exit hook; taking it is atomic, and a claim is never another object's, as a
-# handle the plugin has reused could be. (An entry is also cheaper than a weak reference to each wrapper.)
+# What belongs to a client — buffers, executables and their completion events — refers to it, so a client outlives them
+# while all die by reference count. The garbage collector, though, finalizes the objects of an unreachable cycle (a
+# caught exception's frames, say) in any order, a client before its buffers among them, and a buffer destroyed after its
+# client would return its memory to an allocator that is gone. These objects are therefore tracked by their handle too,
+# and what is left of them is destroyed before the client is. Each object is destroyed by whoever takes its handle out of
+# its one-element claim list — the wrapper's finalizer, its client's or the exit hook; taking it is atomic, and a claim is
+# never another object's, as a handle the plugin has reused could be. The plugin refuses a call on a wrapper whose claim
+# is empty: it has no handle. (An entry is also cheaper than a weak reference to each wrapper.)
 _LIVE_HANDLES: Dict[int, Tuple["Api", str, int, List[int]]] = {}  # id(claim) → api, destroy function, client, claim
 
 
 class _OwnedHandle:
     _destroy = ""
 
-    def _own(self, api: "Api", handle: int, client: int):
-        self.handle = handle
+    def _own(self, api: "Api", handle: int, client: Optional["Client"]):
         self._claim = claim = [handle]
-        _LIVE_HANDLES[id(claim)] = (api, self._destroy, client, claim)
+        _LIVE_HANDLES[id(claim)] = (api, self._destroy, client.handle if client is not None else 0, claim)
+
+    @property
+    def handle(self) -> Optional[int]:
+        claim = self._claim
+        return claim[0] if claim else None
 
     def __del__(self):
         try:
@@ -390,7 +395,6 @@ class _OwnedHandle:
         except (AttributeError, IndexError):  # never owned, or destroyed with its client
             return
         try:
-            self.handle = None
             api, name = _LIVE_HANDLES.pop(id(self._claim))[:2]
             api.destroy(name, handle)
         except Exception:
@@ -793,10 +797,10 @@ class Device:
 class Event(_OwnedHandle):
     """PJRT_Event wrapper (events.rs); `await_` blocks, `on_ready` registers a callback."""
 
-    def __init__(self, api: Api, handle: int, value=None, client: int = 0):
+    def __init__(self, api: Api, handle: int, value=None, client: Optional["Client"] = None):
         if not handle:
             raise PjrtError(ErrorCode.INVALID_ARGUMENT, "the provided PJRT event handle is a null pointer")
-        self.api, self._value = api, value
+        self.api, self.client, self._value = api, client, value
         self._callbacks = []
         self._own(api, handle, client)
 
@@ -828,7 +832,7 @@ class Buffer(_OwnedHandle):
         if not handle:
             raise PjrtError(ErrorCode.INVALID_ARGUMENT, "the provided PJRT buffer handle is a null pointer")
         self.client = client
-        self._own(client.api, handle, client.handle)
+        self._own(client.api, handle, client)
 
     @property
     def api(self) -> Api:
@@ -1052,8 +1056,8 @@ class ExecutionContext(_Owned):
 class Executable(_OwnedHandle, _Owned):
     _destroy = "PJRT_Executable_Destroy"
 
-    def __init__(self, api: Api, handle: int, client: int = 0):
-        self.api = api
+    def __init__(self, api: Api, handle: int, client: Optional["Client"] = None):
+        self.api, self.client = api, client
         self._own(api, handle, client)
 
     def name(self) -> str:
@@ -1151,7 +1155,7 @@ class LoadedExecutable(_OwnedHandle, _Owned):
             raise PjrtError(ErrorCode.INVALID_ARGUMENT, "the provided PJRT loaded executable handle is a null pointer")
         self.client = client
         self._counts, self._local = None, threading.local()
-        self._own(client.api, handle, client.handle)
+        self._own(client.api, handle, client)
 
     @property
     def api(self) -> Api:
@@ -1163,7 +1167,7 @@ class LoadedExecutable(_OwnedHandle, _Owned):
 
     def executable(self) -> Executable:
         a = self.api.call("PJRT_LoadedExecutable_GetExecutable", loaded_executable=self.handle)
-        return Executable(self.api, a.executable, self.client.handle)
+        return Executable(self.api, a.executable, self.client)
 
     def device_assignment(self) -> DeviceAssignment:
         """LoadedExecutable::device_assignment (programs.rs:704-736; decoding as devices.rs:674-688)."""
@@ -1185,7 +1189,8 @@ class LoadedExecutable(_OwnedHandle, _Owned):
                 prepared = self._local.prepared
             except AttributeError:
                 prepared = self._local.prepared = {}
-            key = (launch_id, *[x.handle for x in inputs[0]])
+            # (the executable's own handle among them: the block refers to it)
+            key = (launch_id, self.handle, *[x.handle for x in inputs[0]])
             prep = prepared.get(key)
             if prep is None:
                 if len(prepared) >= 32:
@@ -1197,7 +1202,7 @@ class LoadedExecutable(_OwnedHandle, _Owned):
             if err:
                 raise client.api.error(err)
             return [ExecutionDeviceOutputs([Buffer(client, outs[o]) for o in range(output_count)],
-                                           Event(client.api, events[0], None, client.handle))]
+                                           Event(client.api, events[0], None, client))]
         if len(inputs) != device_count:
             raise PjrtError(ErrorCode.INVALID_ARGUMENT,
                             f"expected inputs for {device_count} device(s) but got inputs for {len(inputs)} device(s)")

@@ -173,3 +173,13 @@ def test_profiler_device_events_time_the_gemm(gpu_client):
         assert 1e6 < e.duration_ps < 5e9  # 1 µs .. 5 ms
     offs = [e.offset_ps for e in gemm]
     assert offs == sorted(offs) and offs[0] >= 0
+
+
+def test_events_keep_their_client(plugin):
+    """The completion event of an execution can be awaited after every other name of its client is gone."""
+    client = plugin.client({"visible_devices": [0]})
+    a = client.buffer(np.array([7, 8], np.int32), pjrt.BufferType.S32, [2, 1])
+    done = client.compile(pjrt.Program.mlir(ADD_PROGRAM)).execute([[a, a]])[0].done
+    del client, a
+    done.await_()
+    assert done.is_ready()

@@ -729,3 +729,30 @@ def test_client_in_a_reference_cycle_outlives_what_it_owns(plugin):
         api._fns.update(real)
         gc.enable()
     assert sorted(order) == sorted(names) and order[-1] == "PJRT_Client_Destroy", order
+
+
+def test_executable_outlives_the_names_of_its_client(plugin):
+    """An executable handed out by a loaded executable keeps the client it belongs to alive."""
+    import gc
+
+    client = plugin.client({"compile_only": True})
+    exe = client.compile(pjrt.Program.mlir(ADD_2X1))
+    inner = exe.executable()
+    del exe, client
+    gc.collect()
+    assert inner.name() == "main" and inner.output_dimensions() == [[2, 1]]
+
+
+def test_a_wrapper_destroyed_with_its_client_refuses_to_be_used(plugin):
+    """What a client took with it (a finalizer may run before those of the wrappers in its cycle) is an error, not a
+    stale handle."""
+    client = plugin.client({"compile_only": True})
+    exe = client.compile(pjrt.Program.mlir(ADD_2X1))
+    inner = exe.executable()
+    client.__del__()
+    assert exe.handle is None and inner.handle is None
+    for call in (inner.name, inner.output_count, exe.addressable_devices, exe.executable, exe.describe_plan,
+                 lambda: exe.execute([[]])):
+        with pytest.raises(pjrt.PjrtError) as e:
+            call()
+        assert e.value.code == pjrt.ErrorCode.INVALID_ARGUMENT and "null" in str(e.value), e.value
