@@ -366,7 +366,7 @@ class _Owned:
         return obj
 
 
-# What belongs to a client — buffers, executables and their completion events — refers to it, so a client outlives them
+# What belongs to a client — buffers, executables and the events of both — refers to it, so a client outlives them
 # while all die by reference count. The garbage collector, though, finalizes the objects of an unreachable cycle (a
 # caught exception's frames, say) in any order, a client before its buffers among them, and a buffer destroyed after its
 # client would return its memory to an allocator that is gone. These objects are therefore tracked by their handle too,
@@ -419,9 +419,9 @@ def _destroy_handles(client: Optional[int] = None):
 
 @atexit.register
 def _destroy_live_objects():
+    _destroy_handles()  # (before the clients they belong to, and events that belong to none, which may wait on one)
     for obj in sorted(list(_LIVE.values()), key=lambda o: o._exit_order):
         obj.__del__()
-    _destroy_handles()
 
 
 class LayoutsExtension:
@@ -869,7 +869,8 @@ class Buffer(_OwnedHandle):
         return [int(t.minor_to_major[i]) for i in range(t.minor_to_major_size)]
 
     def ready_event(self) -> Event:
-        return Event(self.api, self.api.call("PJRT_Buffer_ReadyEvent", buffer=self.handle).event)
+        a = self.api.call("PJRT_Buffer_ReadyEvent", buffer=self.handle)
+        return Event(self.api, a.event, None, self.client)
 
     def memory_layout(self) -> Layout:
         ext = self.api.layouts_extension()
@@ -888,7 +889,7 @@ class Buffer(_OwnedHandle):
         size = self.api.call("PJRT_Buffer_ToHostBuffer", src=self.handle, dst=None).dst_size
         out = (C.c_uint8 * max(size, 1))()
         a = self.api.call("PJRT_Buffer_ToHostBuffer", src=self.handle, dst=C.cast(out, _vp), dst_size=size)
-        return Event(self.api, a.event, lambda: C.string_at(out, size))
+        return Event(self.api, a.event, lambda: C.string_at(out, size), self.client)
 
     def copy_raw_to_host(self, size: int, offset: int = 0) -> Event:
         """Buffer::copy_raw_to_host_buffer (buffers.rs:1318-1340): `size` bytes of the on-device bytes from `offset`;
@@ -896,7 +897,7 @@ class Buffer(_OwnedHandle):
         out = (C.c_uint8 * max(size, 1))()
         a = self.api.call("PJRT_Buffer_CopyRawToHost", buffer=self.handle, dst=C.cast(out, _vp), offset=offset,
                           transfer_size=size)
-        return Event(self.api, a.event, lambda: bytes(out)[:size])
+        return Event(self.api, a.event, lambda: bytes(out)[:size], self.client)
 
     def copy_to_device(self, device: Device) -> "Buffer":
         a = self.api.call("PJRT_Buffer_CopyToDevice", buffer=self.handle, dst_device=device.handle)
@@ -920,7 +921,7 @@ class Buffer(_OwnedHandle):
         if size:
             a = self.api.call("PJRT_Buffer_ToHostBuffer", src=self.handle, dst=C.c_void_p(out.ctypes.data),
                               dst_size=size)
-            Event(self.api, a.event).await_()
+            Event(self.api, a.event, None, self.client).await_()
         return out
 
 
@@ -1241,7 +1242,7 @@ class LoadedExecutable(_OwnedHandle, _Owned):
                       output_lists=out_lists, device_complete_events=events, execute_device=None)
         results = []
         for d in range(device_count):
-            done = Event(self.api, events[d])
+            done = Event(self.api, events[d], None, self.client)
             outs = [Buffer(self.client, out_arrays[d][o]) for o in range(output_count)]
             results.append(ExecutionDeviceOutputs(outs, done))
         return results
@@ -1416,7 +1417,7 @@ class Client(_Owned):
                           device=None, memory=memory.handle, device_layout=None, **kw)
         del keep
         if a.done_with_host_buffer:
-            Event(self.api, a.done_with_host_buffer)  # dropped, as ryft-pjrt does
+            Event(self.api, a.done_with_host_buffer, None, self)  # dropped, as ryft-pjrt does
         return Buffer(self, a.buffer)
 
     def uninitialized_buffer(self, element_type: BufferType, dims: Sequence[int],

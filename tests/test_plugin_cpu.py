@@ -756,3 +756,58 @@ def test_a_wrapper_destroyed_with_its_client_refuses_to_be_used(plugin):
         with pytest.raises(pjrt.PjrtError) as e:
             call()
         assert e.value.code == pjrt.ErrorCode.INVALID_ARGUMENT and "null" in str(e.value), e.value
+
+
+def test_every_event_of_a_client_refers_to_it(plugin, monkeypatch):
+    """Ready events, copies to the host and executions with donated inputs: their events keep the client alive, and are
+    destroyed with it, like those of plain executions. (A compile-only client has no buffers: the plugin's functions
+    are stood in for.)"""
+    client = plugin.client({"compile_only": True})
+    api = plugin.api()
+
+    def event():
+        return api.call("PJRT_Event_Create").event
+
+    def give(field):
+        return lambda ref: setattr(ref._obj, field, event())
+
+    def execute(ref):
+        ref._obj.device_complete_events[0] = event()
+
+    exe = client.compile(pjrt.Program.mlir(ADD_2X1))
+    exe._counts = (1, 0)
+    monkeypatch.setitem(api._fns, "PJRT_Buffer_Destroy", lambda ref: None)
+    monkeypatch.setitem(api._fns, "PJRT_Buffer_ReadyEvent", give("event"))
+    monkeypatch.setitem(api._fns, "PJRT_Buffer_ToHostBuffer", lambda ref: give("event")(ref) if ref._obj.dst else None)
+    monkeypatch.setitem(api._fns, "PJRT_Buffer_CopyRawToHost", give("event"))
+    monkeypatch.setitem(api._fns, "PJRT_LoadedExecutable_Execute", execute)
+    b = pjrt.Buffer(client, 1 << 40)
+    events = [b.ready_event(), b.copy_to_host(), b.copy_raw_to_host(4), exe.execute([[b, b]])[0].done,
+              exe.execute([[pjrt.ExecutionInput(b, donatable=True), pjrt.ExecutionInput(b)]])[0].done]
+    assert all(e.client is client for e in events), events
+    client.__del__()
+    assert all(e.handle is None for e in events), events
+
+
+_EXIT_ORDER_SCRIPT = r'''
+import sys
+sys.path.insert(0, sys.argv[1])
+from ryft_amd import pjrt
+plugin = pjrt.load_plugin()
+api = plugin.api()
+client = plugin.client({"compile_only": True})
+exe = client.compile(pjrt.Program.mlir(sys.argv[2]))
+event = pjrt.Event(api, api.call("PJRT_Event_Create").event)  # of no client
+for n in ("PJRT_Client_Destroy", "PJRT_LoadedExecutable_Destroy", "PJRT_Event_Destroy"):
+    api._fns[n] = lambda ref, n=n, f=api.fn(n): (print(n, flush=True), f(ref))[1]
+'''
+
+
+def test_clients_are_destroyed_last_at_exit():
+    import sys
+    r = subprocess.run([sys.executable, "-c", _EXIT_ORDER_SCRIPT, ROOT, ADD_2X1], capture_output=True, text=True,
+                       timeout=120)
+    assert r.returncode == 0, r.stderr
+    order = r.stdout.split()
+    assert sorted(order) == ["PJRT_Client_Destroy", "PJRT_Event_Destroy", "PJRT_LoadedExecutable_Destroy"], r.stdout
+    assert order[-1] == "PJRT_Client_Destroy", order
