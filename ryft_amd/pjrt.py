@@ -369,12 +369,15 @@ class _Owned:
 # What belongs to a client — buffers, executables and the events of both — refers to it, so a client outlives them
 # while all die by reference count. The garbage collector, though, finalizes the objects of an unreachable cycle (a
 # caught exception's frames, say) in any order, a client before its buffers among them, and a buffer destroyed after its
-# client would return its memory to an allocator that is gone. These objects are therefore tracked by their handle too,
-# and what is left of them is destroyed before the client is. Each object is destroyed by whoever takes its handle out of
-# its one-element claim list — the wrapper's finalizer, its client's or the exit hook; taking it is atomic, and a claim is
-# never another object's, as a handle the plugin has reused could be. The plugin refuses a call on a wrapper whose claim
-# is empty: it has no handle. (An entry is also cheaper than a weak reference to each wrapper.)
-_LIVE_HANDLES: Dict[int, Tuple["Api", str, int, List[int]]] = {}  # id(claim) → api, destroy function, client, claim
+# client would return its memory to an allocator that is gone. Each client therefore lists what belongs to it, by handle,
+# and empties the list before it is destroyed. An object is destroyed by whoever takes its entry out of the list — the
+# wrapper's finalizer, its client's or the exit hook; taking an entry is atomic, also where the garbage collector runs
+# other finalizers meanwhile, and it goes before the object does, so that a handle the plugin uses again finds its place
+# free. An entry shares the wrapper's one-element claim, which holds its handle: once that is empty the wrapper has no
+# handle, and the plugin refuses a call on it. (An entry is cheaper than a weak reference to each wrapper, and unlike a
+# reference to the wrapper's attributes keeps nothing alive.)
+_Belongings = Dict[int, Tuple[str, List[int]]]  # handle → destroy function, claim
+_CLIENTLESS: Dict["Api", _Belongings] = {}  # events that belong to no client
 
 
 class _OwnedHandle:
@@ -382,7 +385,8 @@ class _OwnedHandle:
 
     def _own(self, api: "Api", handle: int, client: Optional["Client"]):
         self._claim = claim = [handle]
-        _LIVE_HANDLES[id(claim)] = (api, self._destroy, client.handle if client is not None else 0, claim)
+        self._siblings = siblings = client._owned if client is not None else _CLIENTLESS.setdefault(api, {})
+        siblings[handle] = (self._destroy, claim)
 
     @property
     def handle(self) -> Optional[int]:
@@ -391,26 +395,22 @@ class _OwnedHandle:
 
     def __del__(self):
         try:
-            handle = self._claim.pop()
-        except (AttributeError, IndexError):  # never owned, or destroyed with its client
-            return
-        try:
-            api, name = _LIVE_HANDLES.pop(id(self._claim))[:2]
-            api.destroy(name, handle)
-        except Exception:
+            claim = self._claim
+            handle = claim[0]
+            if self._siblings.pop(handle, None) is not None:
+                claim.clear()
+                self.api.destroy(self._destroy, handle)
+        except Exception:  # (never owned: AttributeError; destroyed with its client: IndexError)
             pass
 
 
-def _destroy_handles(client: Optional[int] = None):
-    """Destroys the tracked objects of one client (None: of every client)."""
-    for key, (api, name, owner, claim) in list(_LIVE_HANDLES.items()):
-        if client is not None and owner != client:
-            continue
+def _destroy_owned(api: "Api", owned: _Belongings):
+    while True:
         try:
-            handle = claim.pop()
-        except IndexError:
-            continue
-        _LIVE_HANDLES.pop(key, None)
+            handle, (name, claim) = owned.popitem()
+        except KeyError:
+            return
+        claim.clear()
         try:
             api.destroy(name, handle)
         except Exception:
@@ -419,7 +419,8 @@ def _destroy_handles(client: Optional[int] = None):
 
 @atexit.register
 def _destroy_live_objects():
-    _destroy_handles()  # (before the clients they belong to, and events that belong to none, which may wait on one)
+    for api, owned in list(_CLIENTLESS.items()):
+        _destroy_owned(api, owned)
     for obj in sorted(list(_LIVE.values()), key=lambda o: o._exit_order):
         obj.__del__()
 
@@ -1190,8 +1191,11 @@ class LoadedExecutable(_OwnedHandle, _Owned):
                 prepared = self._local.prepared
             except AttributeError:
                 prepared = self._local.prepared = {}
-            # (the executable's own handle among them: the block refers to it)
-            key = (launch_id, self.handle, *[x.handle for x in inputs[0]])
+            try:  # (the executable's own handle among them: the block refers to it)
+                key = (launch_id, self._claim[0], *[x._claim[0] for x in inputs[0]])
+            except IndexError:
+                raise PjrtError(ErrorCode.INVALID_ARGUMENT,
+                                "the executable or an input is null: it was destroyed with its client") from None
             prep = prepared.get(key)
             if prep is None:
                 if len(prepared) >= 32:
@@ -1285,6 +1289,7 @@ class Client(_Owned):
             raise PjrtError(ErrorCode.INVALID_ARGUMENT, "the provided PJRT client handle is a null pointer")
         self.plugin, self.handle = plugin, handle
         self.api = plugin.api()
+        self._owned: _Belongings = {}
 
     @staticmethod
     def _create(plugin: Plugin, options: Dict[str, object]) -> "Client":
@@ -1469,9 +1474,11 @@ class Client(_Owned):
 
     def __del__(self):
         try:
-            if self.handle:
-                _destroy_handles(self.handle)
-                self.api.call("PJRT_Client_Destroy", client=self.handle)
-                self.handle = None
+            handle, self.handle = self.handle, None
+            if handle:
+                try:
+                    _destroy_owned(self.api, self._owned)
+                finally:
+                    self.api.destroy("PJRT_Client_Destroy", handle)
         except Exception:
             pass

@@ -811,3 +811,49 @@ def test_clients_are_destroyed_last_at_exit():
     order = r.stdout.split()
     assert sorted(order) == ["PJRT_Client_Destroy", "PJRT_Event_Destroy", "PJRT_LoadedExecutable_Destroy"], r.stdout
     assert order[-1] == "PJRT_Client_Destroy", order
+
+
+def test_client_is_destroyed_while_the_collector_finalizes_its_objects(plugin, monkeypatch):
+    """Finalizers of other objects of the client run while it destroys what it owns (the collector may run at any
+    allocation): nothing is destroyed twice or left, and the client goes last."""
+    import gc
+
+    api = plugin.api()
+    client = plugin.client({"compile_only": True})
+    exes = [client.compile(pjrt.Program.mlir(ADD_2X1)) for _ in range(3)]
+    destroyed = []
+    for n in ("PJRT_Client_Destroy", "PJRT_LoadedExecutable_Destroy", "PJRT_Executable_Destroy"):
+        monkeypatch.setitem(api._fns, n, lambda ref, n=n, f=api.fn(n): (destroyed.append(n), f(ref))[1])
+    thresholds = gc.get_threshold()
+    gc.collect()
+    gc.disable()
+    try:
+        views = [exes[0].executable() for _ in range(3000)]
+        gc.set_threshold(10 ** 6)
+        for v in views[:50]:  # cyclic garbage, finalized by a collection in the middle of it
+            v.cycle = v
+        del v, views[:50]
+        gc.enable()
+        gc.set_threshold(gc.get_count()[0] + 1000)
+        client.__del__()
+    finally:
+        gc.set_threshold(*thresholds)
+        gc.enable()
+    del exes, views
+    gc.collect()
+    assert len(destroyed) == 3004 and destroyed[-1] == "PJRT_Client_Destroy", (len(destroyed), destroyed[-1])
+
+
+def test_a_callback_that_refers_to_its_event_is_collected(plugin):
+    """The list of a client's objects keeps nothing alive: an event whose callback refers to it is still collected."""
+    import gc
+    import weakref
+
+    client = plugin.client({"compile_only": True})
+    api = plugin.api()
+    event = pjrt.Event(api, api.call("PJRT_Event_Create").event, None, client)
+    event.on_ready(lambda err: event)
+    alive = weakref.ref(event)
+    del event
+    gc.collect()
+    assert alive() is None
