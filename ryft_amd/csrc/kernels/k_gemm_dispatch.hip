@@ -337,7 +337,7 @@ bool gemm_edge_tile(const GemmArgs& a, int* bm, int* bn) {
   return true;
 }
 
-int gemm_plan_splits(const GemmArgs& a) {
+int gemm_plan_splits(const GemmArgs& a, int64_t edge_partials) {
   GemmArgs g = a;
   g.splits = 1;
   Choice c;
@@ -348,7 +348,7 @@ int gemm_plan_splits(const GemmArgs& a) {
     double cost = tile_cost(g, kind, c, 1);
     for (int s = 2; s <= 16; s *= 2) {
       g.splits = s;
-      if (!pick_mfma(g, &c)) continue;
+      if (gemm_partial_bytes(g, s) > edge_partials || !pick_mfma(g, &c)) continue;
       const double t = tile_cost(g, kind, c, s);
       if (t < cost) best = s, cost = t;
     }
@@ -377,7 +377,7 @@ int gemm_plan_splits(const GemmArgs& a) {
   return pick_mfma(g, &c) ? best : 1;
 }
 
-int gemm_plan_family(const GemmArgs& a) {
+int gemm_plan_family(const GemmArgs& a, int64_t edge_partials) {
   // Full tiles where they fit, unless the edge family (smaller tiles, deeper pipelines, more ways to split) is estimated
   // to save a fifth of the time and 6 µs, the estimates' own error. Both sides measured: bf16 1024³ 19.6 µs in full
   // tiles over 4 K ranges, 7.5 in 64×64 tiles; 512 × 4096 × 4096 36 and 28; i8 512 × 4096 × 4096 32.5 and 21.5; f8
@@ -392,7 +392,7 @@ int gemm_plan_family(const GemmArgs& a) {
     g.family = f;
     g.splits = 1;
     if (!pick_mfma(g, &c)) return f == 1 ? 2 : 1;
-    const int s = gemm_plan_splits(g);
+    const int s = gemm_plan_splits(g, edge_partials);
     g.splits = s;
     if (s > 1 && !pick_mfma(g, &c)) return 1;
     cost[f] = tile_cost(g, kind, c, s);

@@ -31,11 +31,16 @@ int gemm_mfma_layout_gaps(const GemmArgs& a);
 const char* gemm_kernel_name(const GemmArgs& a);
 // Whether launch_gemm() runs these arguments on an edge kernel (its name stands for the family), and on which tile.
 bool gemm_edge_tile(const GemmArgs& a, int* bm, int* bn);
-// The tile family (GemmArgs::family) launch_gemm should run these unsplit arguments in.
-int gemm_plan_family(const GemmArgs& a);
-// Number of K ranges launch_gemm splits these arguments into when given a workspace of
-// splits × (dual ? 2 : 1) × batch × M × N 4-byte accumulators (1: no split).
-int gemm_plan_splits(const GemmArgs& a);
+// Bytes of the workspace launch_gemm needs to run these arguments in `splits` K ranges (4-byte accumulators).
+inline int64_t gemm_partial_bytes(const GemmArgs& a, int splits) {
+  return (int64_t)splits * (a.dual ? 2 : 1) * a.batch * a.M * a.N * 4;
+}
+// The tile family (GemmArgs::family) launch_gemm should run these unsplit arguments in, edge tiles taking at most
+// `edge_partials` bytes of partial sums.
+int gemm_plan_family(const GemmArgs& a, int64_t edge_partials);
+// Number of K ranges launch_gemm splits these arguments into when given a workspace of gemm_partial_bytes (1: no
+// split); edge tiles are split as far as `edge_partials` bytes allow.
+int gemm_plan_splits(const GemmArgs& a, int64_t edge_partials);
 // Head dims the fused attention kernel supports.
 bool attention_supported(int head_dim);
 // Why the fused attention kernel cannot run these arguments (null: it can). The planner calls it with the operands'

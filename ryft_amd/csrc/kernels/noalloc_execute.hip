@@ -17,7 +17,7 @@
 namespace ryft {
 namespace {
 
-constexpr size_t kScratchBytes = (size_t)64 << 20;  // 64 MiB per GPU
+constexpr size_t kScratchBytes = kNoAllocScratchBytes;  // 64 MiB per GPU
 constexpr int kMaxDevices = 64;
 constexpr size_t kMaxSlots = 1024;
 
@@ -89,11 +89,8 @@ extern "C" int RyftMi355x_ExecuteNoAlloc(PJRT_LoadedExecutable* executable, cons
   if ((num_inputs && (!inputs || !input_sizes)) || (num_outputs && (!outputs || !output_sizes)))
     return report(PJRT_Error_Code_INVALID_ARGUMENT, "input / output pointer or size array is null");
 
-  // Intermediates, each at a 256-byte aligned offset of the scratch array (the alignment the planner assumes of
-  // every slot's base).
-  size_t need = 0;
-  for (const Slot& sl : plan.slots)
-    if (sl.kind == Slot::TEMP) need += (sl.type.bytes() + 255) & ~(size_t)255;
+  // Intermediates, each at a 256-byte aligned offset of the scratch array.
+  const size_t need = plan.temp_bytes();
   if (need > kScratchBytes)
     return report(PJRT_Error_Code_RESOURCE_EXHAUSTED,
                   "executable needs %zu bytes of intermediates; the allocation-free scratch holds %zu", need,

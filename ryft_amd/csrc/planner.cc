@@ -1785,7 +1785,7 @@ void Planner::emit_dot(const std::vector<int>& dots_in, int target, int root) {
     G.epilogue = EPI_STORE;
     st.patches.push_back({offsetof(GemmArgs, out_ptr), out});
     st.bytes += (double)d.type.bytes();
-    G.family = gemm_plan_family(G);
+    G.family = gemm_plan_family(G, opts_.edge_partials);
     st.name = gemm_kernel_name(G);
     plan_split_k(st);
     plan_.steps.push_back(std::move(st));
@@ -1853,7 +1853,7 @@ void Planner::emit_dot(const std::vector<int>& dots_in, int target, int root) {
       return;
     }
   }
-  G.family = gemm_plan_family(G);
+  G.family = gemm_plan_family(G, opts_.edge_partials);
   st.name = gemm_kernel_name(G);
   plan_split_k(st);
   plan_.steps.push_back(std::move(st));
@@ -1867,7 +1867,7 @@ void Planner::emit_dot(const std::vector<int>& dots_in, int target, int root) {
 void Planner::plan_split_k(Step& st) {
   GemmArgs& G = st.gemm;
   if (G.epilogue == EPI_PROGRAM) return;
-  const int s = gemm_plan_splits(G);
+  const int s = gemm_plan_splits(G, opts_.edge_partials);
   if (s <= 1) return;
   TensorType wt;
   wt.dtype = DType::F32;
@@ -1879,10 +1879,11 @@ void Planner::plan_split_k(Step& st) {
   // their whole traffic then stays short of the tail a reduction launch adds (C1: 2 MiB, 11.2 against 13.5 µs a
   // step). Large ones (C5's down projection: 32 MiB) go to the reduction launch, which reads them with every CU
   // instead of one finishing workgroup per tile (75 against 89 µs).
-  const double partial_bytes = (double)s * (G.dual ? 2 : 1) * G.batch * G.M * G.N * 4.0;
+  const int64_t partial_bytes = gemm_partial_bytes(G, s);
   int bm = 0, bn = 0;
   const bool edge = gemm_edge_tile(G, &bm, &bn);
-  if ((!G.dual || edge) && partial_bytes <= 8.0 * (1 << 20)) {
+  if (edge) plan_.edge_partial_bytes += plan_.slots[ws].type.bytes();
+  if ((!G.dual || edge) && partial_bytes <= 8 << 20) {
     // per-output-tile arrival counters for the in-kernel finish: part of the executable (zeroed once when it is
     // loaded; each launch leaves them at zero), sized for the edge kernel's tile, or for the smallest full tile any
     // split kernel uses (64×64)
@@ -2433,8 +2434,26 @@ std::string Plan::describe() const {
 }
 
 Plan build_plan(const Graph& g, const PlanOptions& opts) {
-  Planner p(g, opts);
-  return p.run();
+  Plan plan = Planner(g, opts).run();
+  // Edge GEMMs take the number of K ranges that is estimated fastest. Where it is their partial sums that would keep the
+  // plan from the allocation-free scratch, they get as many as leave it room, down to none: 168 rows of a SwiGLU block
+  // of 5120 × 12928 need 5.8 MiB of temporaries unsplit, 85 MiB as estimated.
+  const size_t need = plan.temp_bytes(), partials = (size_t)plan.edge_partial_bytes;
+  if (need <= kNoAllocScratchBytes || need - partials > kNoAllocScratchBytes) return plan;
+  for (int64_t room = (int64_t)(kNoAllocScratchBytes - (need - partials)); ; room = room > 1 << 20 ? room / 2 : 0) {
+    PlanOptions tight = opts;
+    tight.edge_partials = std::min(opts.edge_partials, room);
+    Plan p = Planner(g, tight).run();
+    if (p.temp_bytes() <= kNoAllocScratchBytes) return p;
+    if (room == 0) return plan;
+  }
+size_t Plan::temp_bytes() const {
+  size_t n = 0;
+  for (const Slot& s : slots)
+    if (s.kind == Slot::TEMP) n += (s.type.bytes() + 255) & ~(size_t)255;
+  return n;
+}
+
 }
 
 }  // namespace ryft

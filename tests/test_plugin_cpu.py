@@ -857,3 +857,17 @@ def test_a_callback_that_refers_to_its_event_is_collected(plugin):
     del event
     gc.collect()
     assert alive() is None
+
+
+def _swiglu(m, d, f):
+    """The SwiGLU block's program at sizes whose input data would take long to make."""
+    sizes = {"7": m, "11": d, "13": f}
+    return re.sub(r"(?<=[<x])(7|11|13)(?=x)", lambda t: str(sizes[t.group()]),
+                  configs.c5_swiglu_fp8(m=7, d=11, f=13).program)
+
+
+@pytest.mark.parametrize("m,d,f", [(168, 5120, 12928), (130, 8192, 28672), (520, 4096, 14352), (1, 4096, 14336)])
+def test_partial_sums_leave_room_for_the_other_temporaries(compile_client, m, d, f):
+    # K ranges are taken as far as the partial sums fit the 64 MiB that an allocation-free execution has
+    exe, _ = _plan(compile_client, _swiglu(m, d, f))
+    assert exe.executable().memory_statistics()["temp_size_in_bytes"] <= 64 << 20, exe.describe_plan()
