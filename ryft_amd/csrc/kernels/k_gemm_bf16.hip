@@ -13,9 +13,9 @@ bool pick_bf16(const GemmArgs& g, bool ar, bool br, Choice* c) {
     return true;
   }
   const int64_t tiles256 = (int64_t)(g.M / 256) * (g.N / 256) * g.batch;
-  if (fits(256, 256, 64) && tiles256 >= 128 && tiles256 < 192) {
-    // 256×256 tiles that would leave a quarter of the CUs or more idle: twice as many of half the size
-    // (2048 × 4096 × 4096: 128 tiles of 256×256 take 84 µs, 256 of 256×128 59 µs)
+  if (fits(256, 256, 64) && tiles256 >= 128 && 2 * tiles256 <= 256) {
+    // 256×256 tiles that would leave half of the CUs idle: twice as many of half the size, which run in one round, a CU
+    // each (2048 × 4096 × 4096: 128 tiles of 256×256 take 84 µs, 256 of 256×128 59 µs)
     *c = br ? make_choice<MMA_BF16, 256, 128, 64, 4, 2, false, true, false>("gemm_bf16_mfma_256x128")
             : make_choice<MMA_BF16, 256, 128, 64, 4, 2, false, false, false>("gemm_bf16_mfma_256x128");
     return true;

@@ -871,3 +871,18 @@ def test_partial_sums_leave_room_for_the_other_temporaries(compile_client, m, d,
     # K ranges are taken as far as the partial sums fit the 64 MiB that an allocation-free execution has
     exe, _ = _plan(compile_client, _swiglu(m, d, f))
     assert exe.executable().memory_statistics()["temp_size_in_bytes"] <= 64 << 20, exe.describe_plan()
+
+
+@pytest.mark.parametrize("m,k,n,kernel", [(2048, 4096, 4096, "256x128"), (2304, 768, 4096, "256x256"),
+                                          (2560, 4096, 4096, "256x256"), (2816, 512, 4096, "256x256"),
+                                          (1792, 1024, 4096, "128x128")])
+def test_half_tiles_where_they_run_in_one_round(compile_client, m, k, n, kernel):
+    # 128 tiles of 256 x 256 are run as 256 of half the size, one to a compute unit; more of them would take two rounds
+    t = lambda *s: "tensor<" + "".join(f"{d}x" for d in s) + "bf16>"
+    _, kernels = _plan(compile_client, f"""module {{
+  func.func @main(%arg0: {t(m, k)}, %arg1: {t(k, n)}) -> {t(m, n)} {{
+    %0 = stablehlo.dot_general %arg0, %arg1, contracting_dims = [1] x [0] : ({t(m, k)}, {t(k, n)}) -> {t(m, n)}
+    return %0 : {t(m, n)}
+  }}
+}}""")
+    assert kernels[0].startswith("gemm_bf16_mfma_" + kernel), kernels
