@@ -275,7 +275,7 @@ static bool pick_mfma(const GemmArgs& g, Choice* c) {
   // MFMA epilogues implement store / scale / SwiGLU; generic programs run on the generic kernel
   if (g.epilogue == EPI_PROGRAM || (g.dual && g.epilogue != EPI_SWIGLU)) return false;
   int kind = mma_kind(g);
-  if (kind < 0) return false;
+  if (kind < 0 || g.K == 0) return false;  // (an empty contraction: the generic kernel writes the epilogue of 0)
   // output types the MFMA epilogue writes (outputs are whole device allocations, so 16-byte aligned)
   const bool int_acc = kind == MMA_I8;
   if (!mfma_out_supported(g.out_dtype[0], int_acc, g.epilogue, false)) return false;
@@ -310,7 +310,7 @@ int gemm_mfma_layout_gaps(const GemmArgs& a) {
   g.splits = 1;
   if (g.epilogue == EPI_PROGRAM) g.epilogue = EPI_STORE;
   const int kind = mma_kind(g);
-  if (kind < 0 || (g.dual && g.epilogue != EPI_SWIGLU)) return -1;
+  if (kind < 0 || g.K == 0 || (g.dual && g.epilogue != EPI_SWIGLU)) return -1;
   int ar = 0, br = 0;
   unsigned gaps = layout_gaps(g, kind, &ar, &br);
   // K-contiguous operands of the edge kernels are read a vector (8-byte piece for a widened f8 B) at a time up to K
@@ -404,7 +404,7 @@ void launch_gemm(const GemmArgs& g, hipStream_t stream, hipEvent_t done) {
   if (g.M == 0 || g.N == 0 || g.batch == 0) return record_done(done, stream);
   Choice c;
   hipError_t e;
-  if (g.K > 0 && pick_mfma(g, &c)) {
+  if (pick_mfma(g, &c)) {
     // shape invariants the MFMA kernels rely on (checked again here, right before the launch)
     if (!c.edge && (g.M % c.bm || g.N % c.bn)) fail(PJRT_Error_Code_INTERNAL, "gemm tile mismatch");
     if (c.lds > 65536) {

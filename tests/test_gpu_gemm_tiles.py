@@ -130,3 +130,10 @@ def test_infinities_past_the_last_k_stay_out(gpu_client):
         (want, dt), = oracle_outputs(prog, ins)
         got = sh.from_raw(outs[0], dt)
         assert np.isinf(want).all() and (got == want).all()
+
+
+@pytest.mark.parametrize("dt,out", [("bf16", "f32"), ("i8", "i32"), ("f32", "f32")])
+def test_empty_contraction(gpu_client, dt, out):
+    name, prog, ins = dot("k0", (16, 0), (0, 24), dt, out, [1], [0])
+    outs, exe = run_pjrt(gpu_client, prog, ins)
+    assert "gemm_generic" in exe.describe_plan() and outs[0].shape == (16, 24) and not outs[0].any()

@@ -886,3 +886,10 @@ def test_half_tiles_where_they_run_in_one_round(compile_client, m, k, n, kernel)
   }}
 }}""")
     assert kernels[0].startswith("gemm_bf16_mfma_" + kernel), kernels
+
+
+@pytest.mark.parametrize("dt,out", [("bf16", "f32"), ("i8", "i32"), ("f32", "f32")])
+def test_empty_contractions_plan_to_the_kernel_they_run_on(compile_client, dt, out):
+    from tests.edge_programs import dot
+    _, prog, _ = dot("k0", (16, 0), (0, 24), dt, out, [1], [0])
+    assert _plan(compile_client, prog)[1] == ["gemm_generic"]
