@@ -329,6 +329,13 @@ const char* gemm_kernel_name(const GemmArgs& a) {
   return "gemm_generic";
 }
 
+std::string gemm_timing_name(const GemmArgs& a, const std::string& name) {
+  int bm, bn;
+  if (!gemm_edge_tile(a, &bm, &bn)) return name;
+  const std::string tile = name.substr(0, name.rfind('_') + 1) + std::to_string(bm) + "x" + std::to_string(bn);
+  return a.splits > 1 ? tile + "_splitk" + std::to_string(a.splits) : tile;
+}
+
 bool gemm_edge_tile(const GemmArgs& a, int* bm, int* bn) {
   Choice c;
   if (!pick_mfma(a, &c) || !c.edge) return false;

@@ -4,6 +4,8 @@
 
 #include <hip/hip_runtime_api.h>
 
+#include <string>
+
 #include "../kernel_abi.h"
 
 namespace ryft {
@@ -27,8 +29,10 @@ void launch_scatter(const ScatterArgs& a, hipStream_t stream, hipEvent_t done = 
 // Operands of these GEMM arguments (bit 0: A, 1: B, 2: B2) whose layout keeps them from the MFMA kernels (0: the
 // MFMA kernels run them as they are; -1: their element types or epilogue have no MFMA kernel whatever the layout).
 int gemm_mfma_layout_gaps(const GemmArgs& a);
-// Name of the GEMM kernel launch_gemm() picks for these arguments (used for profiling labels).
+// Name of the GEMM kernel launch_gemm() picks for these arguments; the edge kernels of a type share one.
 const char* gemm_kernel_name(const GemmArgs& a);
+// Label of the launch in kernel timings: `name`, or for an edge kernel its family with the tile and the K ranges it runs.
+std::string gemm_timing_name(const GemmArgs& a, const std::string& name);
 // Whether launch_gemm() runs these arguments on an edge kernel (its name stands for the family), and on which tile.
 bool gemm_edge_tile(const GemmArgs& a, int* bm, int* bn);
 // Bytes of the workspace launch_gemm needs to run these arguments in `splits` K ranges (4-byte accumulators).

@@ -1895,7 +1895,7 @@ void Planner::plan_split_k(Step& st) {
     plan_.slots[cs].literal.assign((size_t)ct.bytes(), 0);
     st.patches.push_back({offsetof(GemmArgs, tile_counters), cs});
   }
-  // (an edge kernel's label names its family; the plan's text gives the tile and the ranges)
+  // (an edge kernel's name stands for its family; the plan's text and timing_name give the tile and the ranges)
   st.name = edge ? gemm_kernel_name(G) : std::string(gemm_kernel_name(G)) + "_splitk" + std::to_string(s);
 }
 
@@ -2277,6 +2277,7 @@ Plan Planner::run() {
   for (auto& st : plan_.steps) {
     plan_.total_flops += st.flops;
     plan_.total_bytes += st.bytes;
+    st.timing_name = st.kind == Step::GEMM ? gemm_timing_name(st.gemm, st.name) : st.name;
   }
   plan_aliasing();
   return std::move(plan_);

@@ -19,7 +19,8 @@ struct Slot {
 
 struct Step {
   enum Kind { ELEMENTWISE, REDUCE, GEMM, ATTENTION, COPY, ROW, WINDOW, GATHER, REDUCE_BODY, SCATTER, PACK } kind;
-  std::string name;  // kernel family, for profiling ("gemm_bf16_mfma", "attention_fwd", ...)
+  std::string name;  // kernel family ("gemm_bf16_mfma_256x256", "attention_fwd", ...)
+  std::string timing_name;  // label in kernel timings and profiles: the name, or an edge GEMM's own tile and K ranges
   EwProgram ew;
   ReduceArgs red;
   GemmArgs gemm;

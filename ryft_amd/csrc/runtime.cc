@@ -702,7 +702,7 @@ bool enqueue_steps(Client* c, const Plan& plan, void* const* ptr, hipStream_t st
     recorded |= carry != nullptr;
     StepTiming tm;
     if (timed) {
-      tm.name = step.name;
+      tm.name = step.timing_name;
       tm.flops = step.flops;
       tm.bytes = step.bytes;
       tm.device = device_id;

@@ -137,3 +137,15 @@ def test_empty_contraction(gpu_client, dt, out):
     name, prog, ins = dot("k0", (16, 0), (0, 24), dt, out, [1], [0])
     outs, exe = run_pjrt(gpu_client, prog, ins)
     assert "gemm_generic" in exe.describe_plan() and outs[0].shape == (16, 24) and not outs[0].any()
+
+
+def test_timings_name_the_tile_that_ran(gpu_client):
+    for spec, label in (((1000, 1000, 1000), "gemm_bf16_mfma_edge_64x64"), ((1, 4096, 1032), "gemm_bf16_mfma_edge_32x128_splitk16")):
+        m, k, n = spec
+        name, prog, ins = dot("timed", (m, k), (k, n), "bf16", "f32", [1], [0], seed=60)
+        _, exe = run_pjrt(gpu_client, prog, ins)
+        gpu_client.set_kernel_timing(True)
+        run_pjrt(gpu_client, prog, ins, executable=exe)
+        timing = gpu_client.kernel_timing()
+        gpu_client.set_kernel_timing(False)
+        assert list(timing) == [label], timing
