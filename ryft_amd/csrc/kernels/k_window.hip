@@ -8,6 +8,7 @@
 
 #include <algorithm>
 #include <string>
+#include <type_traits>
 
 #include "../common.h"
 #include "ew_device.h"
@@ -471,14 +472,17 @@ template <> struct PackElem<2> { using T = uint16_t; };
 // Rows that only need another pitch (sf == 1), or, gathered element by element, any strides: a 16-byte chunk of the
 // result per thread. HBM-bound; a row's last chunk is read element by element, so that nothing past it is touched.
 // 4 × [3216, 1812] bf16: 233 µs with its product when the elementwise interpreter copied it an element at a time, 34 now.
-template <int ES>
+// WIDE: more chunks than 32 bits count (an operand of 32 GiB and more), at the cost of a 64-bit division each.
+template <int ES, bool WIDE>
 __global__ void __launch_bounds__(256) pack_rows_kernel(const PackArgs A) {
   using T = typename PackElem<ES>::T;
+  using I = std::conditional_t<WIDE, uint64_t, uint32_t>;
   constexpr int V = 16 / ES;
-  const uint32_t cpr = (uint32_t)A.pitch / V, total = (uint32_t)A.K * cpr;
+  const uint32_t cpr = (uint32_t)A.pitch / V;
+  const I total = (I)A.K * cpr;
   for (int b = blockIdx.y; b < A.batch; b += gridDim.y)
-    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < total; i += gridDim.x * 256) {
-      const uint32_t k = i / cpr, f0 = (i - k * cpr) * V;
+    for (I i = blockIdx.x * 256 + threadIdx.x; i < total; i += gridDim.x * 256) {
+      const uint32_t k = (uint32_t)(i / cpr), f0 = (uint32_t)(i - (I)k * cpr) * V;
       const T* src = (const T*)A.src + (int64_t)b * A.sb + (int64_t)k * A.sk + (int64_t)f0 * A.sf;
       u32x4w v = u32x4w{0, 0, 0, 0};
       if (A.sf == 1 && (int)f0 + V <= A.F) {
@@ -544,9 +548,9 @@ void launch_pack_es(const PackArgs& a, hipStream_t stream, hipEvent_t done) {
     launch_k(done, pack_transpose_kernel<ES>, grid, dim3(256), 0, stream, a);
   } else {
     const int64_t chunks = (int64_t)a.K * (a.pitch * ES / 16);
-    if (chunks > INT32_MAX) fail(PJRT_Error_Code_UNIMPLEMENTED, "dot operand too large to copy");
     const dim3 grid((unsigned)std::min<int64_t>((chunks + 255) / 256, 65536), (unsigned)std::min(a.batch, 65535));
-    launch_k(done, pack_rows_kernel<ES>, grid, dim3(256), 0, stream, a);
+    if (chunks > INT32_MAX) launch_k(done, pack_rows_kernel<ES, true>, grid, dim3(256), 0, stream, a);
+    else launch_k(done, pack_rows_kernel<ES, false>, grid, dim3(256), 0, stream, a);
   }
 }
 

@@ -149,3 +149,42 @@ def test_timings_name_the_tile_that_ran(gpu_client):
         timing = gpu_client.kernel_timing()
         gpu_client.set_kernel_timing(False)
         assert list(timing) == [label], timing
+
+
+def test_operand_of_more_chunks_than_32_bits_count(gpu_client):
+    """34.4 GB of int8 whose rows the loads cannot read: the copy indexes its 2^31 + 2^20 vectors of 16 bytes in 64 bits.
+    The operand, (7k + 3f) mod 64, is computed on the device; one-hot rows pick its first, middle and last rows."""
+    K, F = 1 << 20, 32769
+    t = lambda e: f"tensor<{K}x{F}x{e}>"
+    src = f"""module {{
+  func.func @main() -> {t("i8")} {{
+    %0 = stablehlo.iota dim = 0 : {t("i32")}
+    %1 = stablehlo.iota dim = 1 : {t("i32")}
+    %c = stablehlo.constant dense<7> : {t("i32")}
+    %d = stablehlo.constant dense<3> : {t("i32")}
+    %m = stablehlo.constant dense<63> : {t("i32")}
+    %2 = stablehlo.multiply %0, %c : {t("i32")}
+    %3 = stablehlo.multiply %1, %d : {t("i32")}
+    %4 = stablehlo.add %2, %3 : {t("i32")}
+    %5 = stablehlo.and %4, %m : {t("i32")}
+    %6 = stablehlo.convert %5 : ({t("i32")}) -> {t("i8")}
+    return %6 : {t("i8")}
+  }}
+}}"""
+    made = gpu_client.compile(pjrt.Program.mlir(src)).execute([[]])[0]
+    made.done.await_()
+    rows = [0, 1, K // 2, K - 2, K - 1]
+    a = np.zeros((len(rows), K), np.int8)
+    a[np.arange(len(rows)), rows] = 1
+    lt, ot = f"tensor<{len(rows)}x{K}xi8>", f"tensor<{len(rows)}x{F}xi32>"
+    exe = gpu_client.compile(pjrt.Program.mlir(f"""module {{
+  func.func @main(%arg0: {lt}, %arg1: {t("i8")}) -> {ot} {{
+    %0 = stablehlo.dot_general %arg0, %arg1, contracting_dims = [1] x [0] : ({lt}, {t("i8")}) -> {ot}
+    return %0 : {ot}
+  }}
+}}"""))
+    assert "dot_operand_copy" in exe.describe_plan() and "gemm_i8_mfma_edge" in exe.describe_plan(), exe.describe_plan()
+    out = exe.execute([[gpu_client.buffer(a, pjrt.BufferType.S8, a.shape), made.outputs[0]]])[0]
+    out.done.await_()
+    want = (7 * np.array(rows)[:, None] + 3 * np.arange(F)) & 63
+    assert np.array_equal(out.outputs[0].to_numpy(), want)
