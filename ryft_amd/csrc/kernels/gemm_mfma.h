@@ -444,8 +444,8 @@ struct MfmaCfg {
   static constexpr bool SMALL = BM * BN <= 64 * 128;
   static constexpr int NST = DMA && SMALL ? 4 : DMA && 3 * STAGE_D <= 163840 && 2 * STAGE_D > 163840 / 2 ? 3 : 2;
   static constexpr int STAGE = DMA ? STAGE_D : BM * LDK + NB * BREG;
-  // split-K is compiled in for every tile that a plan splits: all but the 256-row ones
-  static constexpr bool SPLIT = BM * BN * NB <= 128 * 256;
+  // split-K is compiled in for the tiles that a plan may split: all but the 256-row ones
+  static constexpr bool SPLIT = BM < 256;
   static_assert(BK % MK == 0, "BK must be a multiple of the MFMA K");
   static_assert(WTM % 32 == 0 && WTN % 32 == 0, "wave tile must be a multiple of 32");
   // epilogue rounds: the largest number of 32-row tile-rows (dividing TM) whose f32 patches fit in the LDS the two

@@ -87,7 +87,7 @@ __global__ void __launch_bounds__(256) gemm_generic_kernel(const GemmArgs G) {
 // ------------------------------------------------------------------------------------------------ split-K
 // Sums the K ranges' partial accumulators in range order and applies the epilogue (splitk_epilogue_oct, shared with
 // the in-kernel finish of the MFMA kernels, so the two give the same bits). Each thread owns 8 consecutive elements
-// of the result (N is a multiple of 16 on every split-K plan): S (the number of ranges, a template argument so that
+// of the result (N is a multiple of 8 on every split-K plan): S (the number of ranges, a template argument so that
 // every range's two 16-byte loads are in flight together) × 2 loads per accumulator set, then one vector store per
 // output.
 template <bool INT, bool DUAL, int S>
@@ -204,7 +204,7 @@ static bool pick_full(const GemmArgs& g, int kind, bool ar, bool br, Choice* c) 
 // compiled in (at most 16 ranges, 8 of a dual GEMM), and no empty range.
 static bool edge_splittable(const GemmArgs& g, const Choice& c, int splits) {
   const int kt = (g.K + c.bk - 1) / c.bk, per = (kt + splits - 1) / splits;
-  return g.N % 8 == 0 && c.bm * c.bn * (g.dual ? 2 : 1) <= 128 * 256 && splits <= (g.dual ? 8 : 16) &&
+  return g.N % 8 == 0 && c.bm < 256 && splits <= (g.dual ? 8 : 16) &&
          (int64_t)(splits - 1) * per < kt;
 }
 
