@@ -130,10 +130,9 @@ def c4_causal_attention(b=4, h=32, s=2048, d=128, seed=0xC4, mask="GE", fill="0x
     The defaults are BASELINE.json's C4. Variants for tests: `mask` is the comparison direction of row (query) index
     against column (key) index ("GT": a strict mask, query 0 sees no key); `fill` the select's fill for masked
     scores (an MLIR float literal); p_type="f32" feeds the f32 probabilities to the second dot_general directly
-    (f32 × bf16 operands, no convert); mask=None drops the mask (plain softmax attention), and `sk` then sets a key /
-    value length of its own."""
+    (f32 × bf16 operands, no convert); mask=None drops the mask (plain softmax attention); `sk` sets a key / value
+    length of its own."""
     sk = s if sk is None else sk
-    assert sk == s or mask is None
     qt = _t((b, h, s, d), "bf16")
     kt = _t((b, h, sk, d), "bf16")
     sf = _t((b, h, s, sk), "f32")
@@ -187,7 +186,8 @@ def c4_causal_attention(b=4, h=32, s=2048, d=128, seed=0xC4, mask="GE", fill="0x
     ins = [HostInput(hd.f32_to_bf16_bits(hd.normal(seed * 16 + i, (b, h, n, d))), BufferType.BF16, (b, h, n, d))
            for i, n in enumerate((s, sk, sk))]
     # unmasked (k <= q) pairs only
-    flops = 4.0 * b * h * d * s * (s + 1) / 2.0 if mask is not None else 4.0 * b * h * d * s * sk
+    n = min(s, sk)
+    flops = 4.0 * b * h * d * (n * (n + 1) / 2.0 + (s - n) * sk if mask is not None else s * sk)
     return Workload("c4_causal_attention", prog, ins, flops=flops, bytes=2.0 * 4 * b * h * s * d,
                     compute_dtype="bf16", tolerance=2e-2,
                     info={"full_square_flops": 4.0 * b * h * s * s * d, "exps": b * h * s * (s + 1) / 2})

@@ -2243,7 +2243,9 @@ bool Planner::try_attention(int d2, int target, DType out_dtype, int root) {
     plan_.slots[cs].literal.assign((size_t)ct.bytes(), 0);
     st.patches.push_back({offsetof(AttnArgs, counters), cs});
   }
-  double pairs = causal ? (double)Sq * (double)(Sk + 1) / 2.0 : (double)Sq * (double)Sk;  // Sq == Sk for causal
+  // causal (k <= q): the queries up to the last key see one key more each, the rest see all
+  const double n = (double)std::min(Sq, Sk);
+  const double pairs = causal ? n * (n + 1) / 2.0 + ((double)Sq - n) * (double)Sk : (double)Sq * (double)Sk;
   st.flops = 4.0 * (double)B * (double)H * (double)Dh * pairs;
   st.bytes = (double)(Qt.bytes() + Kt.bytes() + Vt.bytes() + rn.type.bytes());
   plan_.steps.push_back(std::move(st));

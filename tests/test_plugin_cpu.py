@@ -893,3 +893,13 @@ def test_empty_contractions_plan_to_the_kernel_they_run_on(compile_client, dt, o
     from tests.edge_programs import dot
     _, prog, _ = dot("k0", (16, 0), (0, 24), dt, out, [1], [0])
     assert _plan(compile_client, prog)[1] == ["gemm_generic"]
+
+
+@pytest.mark.parametrize("s,sk", [(130, 200), (200, 130), (70, 70)])
+def test_causal_attention_counts_the_visible_pairs(compile_client, s, sk):
+    w = configs.c4_causal_attention(b=1, h=2, s=s, sk=sk, d=64)
+    exe, kernels = _plan(compile_client, w.program)
+    assert kernels == ["attention_edge"]
+    pairs = sum(min(q + 1, sk) for q in range(s))
+    assert w.flops == 4.0 * 2 * 64 * pairs
+    assert exe.executable().cost_analysis()["flops"] == w.flops
