@@ -2277,9 +2277,9 @@ Plan Planner::run() {
     if (!op_is_elementwise(g_.nodes[g_.results[i]].op)) order.push_back(i);
   for (size_t i : order) materialize(g_.results[i], plan_.output_slots[i]);
   for (auto& st : plan_.steps) {
+    st.timing_name = st.kind == Step::GEMM ? gemm_timing_name(st.gemm, st.name) : st.name;
     plan_.total_flops += st.flops;
     plan_.total_bytes += st.bytes;
-    st.timing_name = st.kind == Step::GEMM ? gemm_timing_name(st.gemm, st.name) : st.name;
   }
   plan_aliasing();
   return std::move(plan_);
@@ -2436,6 +2436,13 @@ std::string Plan::describe() const {
   return os.str();
 }
 
+size_t Plan::temp_bytes() const {
+  size_t n = 0;
+  for (const Slot& s : slots)
+    if (s.kind == Slot::TEMP) n += (s.type.bytes() + 255) & ~(size_t)255;
+  return n;
+}
+
 Plan build_plan(const Graph& g, const PlanOptions& opts) {
   Plan plan = Planner(g, opts).run();
   // Edge GEMMs take the number of K ranges that is estimated fastest. Where it is their partial sums that would keep the
@@ -2450,13 +2457,6 @@ Plan build_plan(const Graph& g, const PlanOptions& opts) {
     if (p.temp_bytes() <= kNoAllocScratchBytes) return p;
     if (room == 0) return plan;
   }
-size_t Plan::temp_bytes() const {
-  size_t n = 0;
-  for (const Slot& s : slots)
-    if (s.kind == Slot::TEMP) n += (s.type.bytes() + 255) & ~(size_t)255;
-  return n;
-}
-
 }
 
 }  // namespace ryft

@@ -66,19 +66,19 @@ struct Plan {
   std::vector<int> output_alias;
   std::vector<bool> output_in_place;
   double total_flops = 0, total_bytes = 0;
-  std::string describe() const;
   int64_t edge_partial_bytes = 0;  // temporaries that hold the partial sums of split edge GEMMs
   // Device memory of the temporaries, each at a 256-byte aligned offset (the alignment the steps assume of a slot).
   size_t temp_bytes() const;
+  std::string describe() const;
 };
 
-struct PlanOptions {
 // Device memory per GPU that an allocation-free execution has for a plan's temporaries.
 constexpr size_t kNoAllocScratchBytes = (size_t)64 << 20;
 
+struct PlanOptions {
   bool fast_paths = true;  // recognise programs that specialised kernels compute (row norm); false: interpret them
-};
   int64_t edge_partials = INT64_MAX;  // most bytes of partial sums that one edge GEMM may take
+};
 Plan build_plan(const Graph& g, const PlanOptions& opts = PlanOptions());
 
 }  // namespace ryft
