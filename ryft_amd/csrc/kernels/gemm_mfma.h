@@ -16,8 +16,9 @@
 // Measured (kernel times, before: register-staged edge tiles of 128×128 only, loads issued behind a branch):
 // 1000³ bf16 17.3 → 8.4 µs (64×64 tiles), Xᵀ·dY of [2048, 4096]ᵀ·[2048, 4096] 103 → 59 µs (256×256, both operands by
 // transposing reads), 16 rows × f8 weights [4096, 14336] twice 77 → 30 µs and [14336, 4096] 172 → 18 µs (32×128 tiles
-// over K ranges). What bounds them: the small tiles the L2-to-LDS rate (about 60 GB/s per CU), the large ones the MFMA
-// issue at the clock the chip holds.
+// over K ranges). What bounds them: the 64×64 tiles the L2-to-LDS rate (about 60 GB/s per CU), the 32×128 tiles of f8 weights
+// the latency of their loads, a barrier per k-tile with too few bytes in flight (16 rows: gate and up 4.7 TB/s from HBM,
+// down 3.7, MFMA busy 12-16%, no LDS queue), the large ones the MFMA issue at the clock the chip holds.
 //
 // Instruction per compute type (all dense, f32 or i32 accumulation):
 //   bf16  v_mfma_f32_32x32x16_bf16      f16  v_mfma_f32_32x32x16_f16
@@ -444,8 +445,6 @@ struct MfmaCfg {
   static constexpr bool SMALL = BM * BN <= 64 * 128;
   static constexpr int NST = DMA && SMALL ? 4 : DMA && 3 * STAGE_D <= 163840 && 2 * STAGE_D > 163840 / 2 ? 3 : 2;
   static constexpr int STAGE = DMA ? STAGE_D : BM * LDK + NB * BREG;
-  // split-K is compiled in for the tiles that a plan may split: all but the 256-row ones
-  static constexpr bool SPLIT = BM < 256;
   static_assert(BK % MK == 0, "BK must be a multiple of the MFMA K");
   static_assert(WTM % 32 == 0 && WTN % 32 == 0, "wave tile must be a multiple of 32");
   // epilogue rounds: the largest number of 32-row tile-rows (dividing TM) whose f32 patches fit in the LDS the two
@@ -817,7 +816,10 @@ __device__ __forceinline__ void epi_round(const GemmArgs& G, int b, int m0, int 
 // EDGE: any M, N (partial tiles at the edges: bounded or clamped loads, masked stores) and any K that is a multiple of
 // the 16-byte vector of each K-contiguous operand (the last k-tile multiplies zeros past K); split-K with N a multiple
 // of 8.
-template <int KIND, int BM, int BN, int BK, int WM, int WN, bool A_R, bool B_R, bool DUAL, bool EDGE>
+// SPLIT: split-K is compiled in (G.splits may be > 1). Edge kernels exist both ways: the finish holds up to 128 registers
+// of partial sums, and with it in the unsplit kernel a SIMD held 2 waves of the f32 64×64 tile instead of 8 (46 and 154
+// registers; 4352 × 2424 × 704 151 and 175 µs).
+template <int KIND, int BM, int BN, int BK, int WM, int WN, bool A_R, bool B_R, bool DUAL, bool EDGE, bool SPLIT>
 __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const GemmArgs G) {
   using C = MfmaCfg<KIND, BM, BN, BK, WM, WN, A_R, B_R, DUAL, EDGE>;
   using M = typename C::M;
@@ -841,7 +843,7 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const GemmArgs 
   // the tiles of that range fetch only its slices of A and B (with the range inside the XCD's run every XCD would
   // fetch the whole of A). A split finished in-kernel (small partial sums) keeps every K range of a tile on the
   // tile's XCD instead, so that the finishing range reads partial sums written on its own XCD.
-  const int nsplit = G.splits > 1 ? G.splits : 1;
+  const int nsplit = SPLIT && G.splits > 1 ? G.splits : 1;
   int split, bid;
   if (nsplit > 1 && G.tile_counters) {
     split = (int)blockIdx.x / total;
@@ -1420,8 +1422,8 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const GemmArgs 
     // moving the reads above the writes is all the ordering needed (a memory fence would also wait for the stores).
     __asm__ __volatile__("" ::: "memory");
     const int em0 = m0 + wm * C::WTM + round * EPI_ROWS * 32, en0 = n0 + wn * C::WTN;
-    if (C::SPLIT && G.splits > 1) {  // raw partial sums of this K range
-      if constexpr (C::SPLIT) {
+    if (SPLIT && G.splits > 1) {  // raw partial sums of this K range
+      if constexpr (SPLIT) {
         constexpr int PDT = M::INT ? DT_S32 : DT_F32;
         const int64_t slice = (int64_t)G.batch * G.M * G.N * 4;
         char* ws = (char*)G.ws + (int64_t)split * C::NB * slice;
@@ -1446,7 +1448,7 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const GemmArgs 
   // counts its arrival at the tile; the last of the S ranges to arrive sums them all and applies the epilogue. No
   // workgroup waits for another, and no cache is flushed or invalidated (the partials are written and read at
   // device scope); the counter is back at zero when the launch ends.
-  if constexpr (C::SPLIT) {
+  if constexpr (SPLIT) {
     if (G.splits > 1 && G.tile_counters) {
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
@@ -1476,6 +1478,7 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const GemmArgs 
 // ------------------------------------------------------------------------------------------------ dispatch
 struct Choice {
   const void* fn = nullptr;
+  const void* split_fn = nullptr;  // the kernel that runs K ranges (null: none does)
   int threads = 256;
   int lds = 0;
   int bm = 0, bn = 0, bk = 0;
@@ -1487,7 +1490,9 @@ template <int KIND, int BM, int BN, int BK, int WM, int WN, bool A_R, bool B_R, 
 Choice make_choice(const char* name) {
   using C = MfmaCfg<KIND, BM, BN, BK, WM, WN, A_R, B_R, DUAL, EDGE>;
   Choice c;
-  c.fn = (const void*)&gemm_mfma_kernel<KIND, BM, BN, BK, WM, WN, A_R, B_R, DUAL, EDGE>;
+  constexpr bool SPLIT = BM < 256;  // (no plan splits the 256-row tiles)
+  c.fn = (const void*)&gemm_mfma_kernel<KIND, BM, BN, BK, WM, WN, A_R, B_R, DUAL, EDGE, SPLIT && !EDGE>;
+  if constexpr (SPLIT) c.split_fn = (const void*)&gemm_mfma_kernel<KIND, BM, BN, BK, WM, WN, A_R, B_R, DUAL, EDGE, true>;
   c.edge = EDGE;
   c.threads = C::THREADS;
   c.lds = C::LDS_BYTES;

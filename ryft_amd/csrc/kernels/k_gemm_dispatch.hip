@@ -204,7 +204,7 @@ static bool pick_full(const GemmArgs& g, int kind, bool ar, bool br, Choice* c) 
 // compiled in (at most 16 ranges, 8 of a dual GEMM), and no empty range.
 static bool edge_splittable(const GemmArgs& g, const Choice& c, int splits) {
   const int kt = (g.K + c.bk - 1) / c.bk, per = (kt + splits - 1) / splits;
-  return g.N % 8 == 0 && c.bm < 256 && splits <= (g.dual ? 8 : 16) &&
+  return g.N % 8 == 0 && c.split_fn && splits <= (g.dual ? 8 : 16) &&
          (int64_t)(splits - 1) * per < kt;
 }
 
@@ -414,11 +414,13 @@ void launch_gemm(const GemmArgs& g, hipStream_t stream, hipEvent_t done) {
   if (pick_mfma(g, &c)) {
     // shape invariants the MFMA kernels rely on (checked again here, right before the launch)
     if (!c.edge && (g.M % c.bm || g.N % c.bn)) fail(PJRT_Error_Code_INTERNAL, "gemm tile mismatch");
+    const int splits = g.splits > 1 ? g.splits : 1;
+    const void* const fn = splits > 1 ? c.split_fn : c.fn;
+    if (!fn) fail(PJRT_Error_Code_INTERNAL, "split-K on a tile that has none");
     if (c.lds > 65536) {
-      e = hipFuncSetAttribute(c.fn, hipFuncAttributeMaxDynamicSharedMemorySize, c.lds);
+      e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, c.lds);
       if (e != hipSuccess) fail(PJRT_Error_Code_INTERNAL, std::string("LDS attribute failed: ") + hipGetErrorString(e));
     }
-    const int splits = g.splits > 1 ? g.splits : 1;
     if (splits > 1 && (!g.ws || (c.edge ? !edge_splittable(g, c, splits) : g.K % (splits * 16) || g.N % 16)))
       fail(PJRT_Error_Code_INTERNAL, "split-K without a workspace or over partial ranges");
     if (splits > 1 && g.tile_counters && ((g.dual && (!c.edge || splits > 8)) || (splits & (splits - 1)) || splits > 16))
@@ -430,9 +432,9 @@ void launch_gemm(const GemmArgs& g, hipStream_t stream, hipEvent_t done) {
     const bool reduce = splits > 1 && !g.tile_counters;
     hipEvent_t main_done = reduce ? nullptr : done;
     hipEvent_t start = take_start();
-    e = main_done || start ? hipExtLaunchKernel(c.fn, dim3((unsigned)blocks), dim3(c.threads), args, (size_t)c.lds,
+    e = main_done || start ? hipExtLaunchKernel(fn, dim3((unsigned)blocks), dim3(c.threads), args, (size_t)c.lds,
                                                 stream, start, main_done, 0)
-                           : hipLaunchKernel(c.fn, dim3((unsigned)blocks), dim3(c.threads), args, (size_t)c.lds, stream);
+                           : hipLaunchKernel(fn, dim3((unsigned)blocks), dim3(c.threads), args, (size_t)c.lds, stream);
     if (e == hipSuccess && reduce) {
       if (g.acc_is_int) launch_splitk_reduce<true, false>(g, stream, done);
       else if (g.dual) launch_splitk_reduce<false, true>(g, stream, done);

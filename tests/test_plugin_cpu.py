@@ -903,3 +903,19 @@ def test_causal_attention_counts_the_visible_pairs(compile_client, s, sk):
     pairs = sum(min(q + 1, sk) for q in range(s))
     assert w.flops == 4.0 * 2 * 64 * pairs
     assert exe.executable().cost_analysis()["flops"] == w.flops
+
+
+def test_unsplit_edge_kernels_hold_no_partial_sums():
+    """The split-K finish keeps up to 128 registers of partial sums; compiled into the unsplit edge kernel of the f32 tile it
+    left a SIMD 2 waves of 8."""
+    csrc = os.path.join(ROOT, "ryft_amd", "csrc")
+    flags = [f for f in re.search(r"HIPFLAGS := (.*)", open(os.path.join(csrc, "Makefile")).read()).group(1).split()
+             if f != "$(COMMON)"]
+    r = subprocess.run(["/opt/rocm/bin/hipcc", "-O3", "-std=c++17", "-I" + os.path.join(ROOT, "include"), "-I" + csrc, *flags,
+                        "--offload-device-only", "-Rpass-analysis=kernel-resource-usage", "-c",
+                        os.path.join(csrc, "kernels", "k_gemm_f32.hip"), "-o", os.devnull],
+                       capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stderr[-2000:]
+    waves = dict(re.findall(r"Function Name: (\S+).*?Occupancy \[waves/SIMD\]: (\d+)", r.stderr, re.S))
+    unsplit = [int(n) for name, n in waves.items() if "ELb1ELb0EEEv" in name]  # edge, not split
+    assert len(unsplit) == 4 and min(unsplit) >= 7, waves
