@@ -970,7 +970,8 @@ __global__ void __launch_bounds__(VNT) rownorm_block_kernel(const RowArgs A) {
 // t of a row's G owns elements t, t + G, ..., eight in flight at a time (loads past the row's end re-read its last
 // element, unused), every access of a wavefront one run of 64 elements. Folded in the order of the interpreted row
 // kernel for such rows (same G, same bits), which it replaces there: interpreting the program element by element was
-// bound by its own instructions, not by memory or latency. The scaling pass reads the row again, from L2.
+// bound by its own instructions, not by memory or latency. The scaling pass reads the row again, mostly past the L2 where
+// the rows in flight exceed it (4000 × 16377: 387 MB for 262 MB of rows).
 // bf16 passes on the host's clock, interpreted → here: 1 × 16383 498 → 13 µs, 170 × 1001 148 → 13, 4000 × 16377
 // 2543 → 76 (3.4 TB/s). What bounds it: few rows the launch and the chain of loads, many rows the 2-byte accesses.
 template <int G>

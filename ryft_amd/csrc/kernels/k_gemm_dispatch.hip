@@ -208,12 +208,57 @@ static bool edge_splittable(const GemmArgs& g, const Choice& c, int splits) {
          (int64_t)(splits - 1) * per < kt;
 }
 
-// Microseconds of one k-tile (128 bytes of k per row; 64 for f32) of a tile: `alone`, of a workgroup with a CU to
-// itself, and `shared`, per workgroup of a busy CU. Measured at (M, K, N) = (1, 4096, 4096), (16, 4096, 14336),
-// (64, 4096, 4096), (300, 4096, 8192), (512, 4096, 4096), (1000, 1000, 1000), (2000, 3000, 4000) and others, every tile
-// and split of each: small tiles move more operand bytes per product (a 64×64 tile's k-tile takes 0.2-0.27 µs whether
-// the CU runs one or eight of them: it is the L2-to-LDS rate, about 60 GB/s per CU) but there are more of them to fill
-// the chip with, and their four LDS stages hide the load latency that two stages of a 128×128 tile alone on a CU do not.
+// What an edge tile's time is made of, in microseconds: a k-tile (128 bytes of k per row; 64 for f32) of a workgroup with a
+// CU to itself (`alone`) and per workgroup of a busy CU (`shared`), a workgroup's start and end (`round`), and storing 16384
+// bytes of its results (`store`). Fitted to the kernel times of 1950 products of drawn shapes (1 to 16000 rows, k 16 to 16000, up to
+// 16 at a time), every tile and number of K ranges of each, then adjusted where the choice was not the best one. Over those
+// shapes the choice takes 1.014 times the best one's time; 1.038 by the family's estimates below, which know neither the
+// results' bytes nor a workgroup's start (64×128 tiles stored the two results of 760 × 896 × 7936 i8 in 26 µs, 128×128 in
+// 21; f32 was split where it fills the chip, 16 × 3328 × 1264 × 48 132 µs, 103 unsplit). Small tiles move more operand bytes
+// per product (a 64×64 tile's k-tile takes 0.2 µs whether the CU runs one or eight of them: it is the L2-to-LDS rate, about
+// 70 GB/s per CU) but there are more of them to fill the chip with, and their four LDS stages hide the load latency that two
+// stages of a 128×128 tile alone on a CU do not.
+struct EdgeTime {
+  int kind, bm, bn, dual;
+  double alone, shared, round, store;
+};
+static constexpr EdgeTime kEdgeTimes[] = {
+    {MMA_BF16, 256, 256, 0, 1.14, 1.28, 2.56, 0.29},     {MMA_BF16, 128, 128, 0, 0.85, 0.50, 1.49, 0.20},
+    {MMA_BF16, 64, 64, 0, 0.26, 0.23, 0.89, 0.00},       {MMA_BF16, 32, 128, 0, 0.06, 0.24, 1.31, 0.00},
+    {MMA_F16, 128, 128, 0, 0.52, 0.44, 1.25, 0.47},      {MMA_F32, 64, 64, 0, 0.44, 0.36, 0.77, 0.12},
+    {MMA_I8, 256, 256, 0, 1.16, 1.17, 3.81, 0.38},       {MMA_I8, 128, 128, 0, 0.70, 0.42, 1.94, 0.43},
+    {MMA_I8, 64, 128, 0, 0.31, 0.40, 1.50, 0.51},        {MMA_I8, 32, 128, 0, 0.25, 0.24, 1.16, 0.26},
+    {MMA_FP8, 128, 128, 0, 0.68, 0.34, 1.24, 0.24},      {MMA_FP8, 128, 128, 1, 1.02, 0.84, 5.01, 0.45},
+    {MMA_BF16_F8, 128, 128, 0, 0.75, 0.47, 1.21, 0.04},  {MMA_BF16_F8, 64, 128, 0, 0.38, 0.25, 1.35, 0.00},
+    {MMA_BF16_F8, 32, 128, 0, 0.22, 0.18, 0.68, 0.00},   {MMA_BF16_F8, 128, 128, 1, 1.02, 0.84, 5.01, 0.45},
+    {MMA_BF16_F8, 64, 128, 1, 0.53, 0.60, 4.01, 0.16},   {MMA_BF16_F8, 32, 128, 1, 0.44, 0.35, 3.03, 0.00}};
+
+// Estimated microseconds of an edge tile over `splits` K ranges: the busiest CU's workgroups, and for a split the reduction
+// launch, or (partial sums up to 8 MiB) the arrival and the finish, in which one workgroup sums and stores a tile by itself:
+// 5.5 µs for 128×128 elements, 17 with a scaled or SwiGLU epilogue.
+static double edge_cost(const GemmArgs& g, int kind, const Choice& c, int splits) {
+  const EdgeTime* t = nullptr;
+  for (const EdgeTime& x : kEdgeTimes)
+    if (x.kind == kind && x.bm == c.bm && x.bn == c.bn && x.dual == (g.dual ? 1 : 0)) t = &x;
+  const double wgs = (double)((g.M + c.bm - 1) / c.bm) * ((g.N + c.bn - 1) / c.bn) * g.batch * splits;
+  if (!t) return wgs * g.K;
+  const int kt = (g.K + c.bk - 1) / c.bk, per = (kt + splits - 1) / splits;
+  const double busiest = std::ceil(wgs / 256);
+  const int result = (int)(dtype_size((DType)g.out_dtype[0]) + (g.raw_out ? dtype_size((DType)g.out_dtype[1]) : 0));
+  const double area = (double)std::min(g.M, c.bm) * std::min(g.N, c.bn) / 16384;
+  const double stored = area * (splits > 1 ? (g.dual ? 8 : 4) : result);
+  double us = 2.4 + per * std::max(t->alone, t->shared * busiest) + busiest * (t->round + t->store * stored);
+  if (splits > 1) {
+    const double mb = (double)gemm_partial_bytes(g, splits) / (1 << 20);
+    us += mb <= 8.0 ? 1.8 + 0.34 * mb + area * (g.epilogue == EPI_STORE ? 5.5 : 16.7) : 6.6 + 0.24 * mb;
+  }
+  return us;
+}
+
+// The choice between the families: microseconds of one k-tile of a tile, `alone`, of a workgroup with a CU to itself, and
+// `shared`, per workgroup of a busy CU. Measured at (M, K, N) = (1, 4096, 4096), (16, 4096, 14336), (64, 4096, 4096),
+// (300, 4096, 8192), (512, 4096, 4096), (1000, 1000, 1000), (2000, 3000, 4000) and others, every tile and split of each.
+// The margins in gemm_plan_family go with these estimates, of full and edge tiles alike.
 struct TileTime {
   int kind, bm, bn, dual;
   double alone, shared;
@@ -228,7 +273,7 @@ static constexpr TileTime kTileTimes[] = {
     {MMA_BF16_F8, 32, 128, 0, 0.28, 0.25}, {MMA_BF16_F8, 256, 128, 1, 1.33, 1.6},  {MMA_BF16_F8, 128, 128, 1, 1.3, 1.0},
     {MMA_BF16_F8, 64, 128, 1, 0.66, 0.65}, {MMA_BF16_F8, 32, 128, 1, 0.6, 0.45}};
 
-// Estimated microseconds of a tile over `splits` K ranges: the k-tiles of the busiest CU's workgroups, and for a
+// Microseconds of a tile over `splits` K ranges as the families are compared: the k-tiles of the busiest CU's workgroups, and for a
 // split the arrival and finish in-kernel (partial sums up to 8 MiB) or the reduction launch, both growing with the
 // partial sums' traffic.
 static double tile_cost(const GemmArgs& g, int kind, const Choice& c, int splits) {
@@ -247,23 +292,28 @@ static double tile_cost(const GemmArgs& g, int kind, const Choice& c, int splits
   return us;
 }
 
+// The edge kernels of these arguments, in `t` (room for 4).
+static int edge_tiles(const GemmArgs& g, int kind, bool ar, bool br, Choice* t) {
+  switch (kind) {
+    case MMA_BF16: return edge_tiles_bf16(g, ar, br, t);
+    case MMA_F16: return edge_tiles_f16(g, ar, br, t);
+    case MMA_I8: return edge_tiles_i8(g, ar, br, t);
+    case MMA_FP8: return edge_tiles_fp8(g, ar, br, t);
+    case MMA_F32: return edge_tiles_f32(g, ar, br, t);
+    case MMA_BF16_F8: return edge_tiles_bf16f8(g, ar, br, t);
+    default: return 0;
+  }
+}
+
 // The edge kernel for these arguments (g.splits K ranges): the candidate whose estimated time is lowest.
 static bool pick_edge_tile(const GemmArgs& g, int kind, bool ar, bool br, Choice* c) {
   Choice t[4];
-  int n = 0;
-  switch (kind) {
-    case MMA_BF16: n = edge_tiles_bf16(g, ar, br, t); break;
-    case MMA_F16: n = edge_tiles_f16(g, ar, br, t); break;
-    case MMA_I8: n = edge_tiles_i8(g, ar, br, t); break;
-    case MMA_FP8: n = edge_tiles_fp8(g, ar, br, t); break;
-    case MMA_F32: n = edge_tiles_f32(g, ar, br, t); break;
-    case MMA_BF16_F8: n = edge_tiles_bf16f8(g, ar, br, t); break;
-  }
+  const int n = edge_tiles(g, kind, ar, br, t);
   int best = -1;
   const int splits = std::max(1, (int)g.splits);
   for (int i = 0; i < n; ++i) {
     if (g.splits > 1 && !edge_splittable(g, t[i], g.splits)) continue;
-    if (best < 0 || tile_cost(g, kind, t[i], splits) < tile_cost(g, kind, t[best], splits)) best = i;
+    if (best < 0 || edge_cost(g, kind, t[i], splits) < edge_cost(g, kind, t[best], splits)) best = i;
   }
   if (best < 0) return false;
   *c = t[best];
@@ -352,11 +402,11 @@ int gemm_plan_splits(const GemmArgs& a, int64_t edge_partials) {
   if (c.edge) {
     int best = 1;
     const int kind = mma_kind(g);
-    double cost = tile_cost(g, kind, c, 1);
+    double cost = edge_cost(g, kind, c, 1);
     for (int s = 2; s <= 16; s *= 2) {
       g.splits = s;
       if (gemm_partial_bytes(g, s) > edge_partials || !pick_mfma(g, &c)) continue;
-      const double t = tile_cost(g, kind, c, s);
+      const double t = edge_cost(g, kind, c, s);
       if (t < cost) best = s, cost = t;
     }
     return best;
@@ -393,18 +443,25 @@ int gemm_plan_family(const GemmArgs& a, int64_t edge_partials) {
   GemmArgs g = a;
   g.splits = 1;
   const int kind = mma_kind(g);
-  double cost[3] = {0, 0, 0};
-  for (int f = 1; f <= 2; ++f) {
-    Choice c;
-    g.family = f;
-    g.splits = 1;
-    if (!pick_mfma(g, &c)) return f == 1 ? 2 : 1;
-    const int s = gemm_plan_splits(g, edge_partials);
-    g.splits = s;
-    if (s > 1 && !pick_mfma(g, &c)) return 1;
-    cost[f] = tile_cost(g, kind, c, s);
-  }
-  return cost[2] < 0.8 * cost[1] && cost[2] < cost[1] - 6.0 ? 2 : 1;
+  Choice c;
+  g.family = 1;
+  if (!pick_mfma(g, &c)) return 2;
+  g.splits = gemm_plan_splits(g, edge_partials);
+  if (g.splits > 1 && !pick_mfma(g, &c)) return 1;
+  const double full = tile_cost(g, kind, c, g.splits);
+  g.family = 2;
+  g.splits = 1;
+  if (!pick_mfma(g, &c)) return 1;
+  int ar = 0, br = 0;
+  layout_gaps(g, kind, &ar, &br);
+  Choice t[4];
+  const int n = edge_tiles(g, kind, ar, br, t);
+  double edge = HUGE_VAL;
+  for (int s = 1; s <= 16; s *= 2)
+    for (int i = 0; i < n; ++i)
+      if (s == 1 || (gemm_partial_bytes(g, s) <= edge_partials && edge_splittable(g, t[i], s)))
+        edge = std::min(edge, tile_cost(g, kind, t[i], s));
+  return edge < 0.8 * full && edge < full - 6.0 ? 2 : 1;
 }
 
 void launch_gemm(const GemmArgs& g, hipStream_t stream, hipEvent_t done) {

@@ -866,10 +866,23 @@ def _swiglu(m, d, f):
                   configs.c5_swiglu_fp8(m=7, d=11, f=13).program)
 
 
-@pytest.mark.parametrize("m,d,f", [(168, 5120, 12928), (130, 8192, 28672), (520, 4096, 14352), (1, 4096, 14336)])
-def test_partial_sums_leave_room_for_the_other_temporaries(compile_client, m, d, f):
+def _bf16_dot(b, m, k, n):
+    t = lambda *s: "tensor<" + "".join(f"{d}x" for d in s) + "bf16>"
+    l, r, o = t(b, m, k), t(b, k, n), t(b, m, n)
+    return f"""module {{
+  func.func @main(%arg0: {l}, %arg1: {r}) -> {o} {{
+    %0 = stablehlo.dot_general %arg0, %arg1, batching_dims = [0] x [0], contracting_dims = [2] x [1] : ({l}, {r}) -> {o}
+    return %0 : {o}
+  }}
+}}"""
+
+
+@pytest.mark.parametrize("program", [lambda: _swiglu(168, 5120, 12928), lambda: _swiglu(130, 8192, 28672),
+                                     lambda: _swiglu(520, 4096, 14352), lambda: _swiglu(1, 4096, 14336),
+                                     lambda: _bf16_dot(16, 2432, 11520, 128), lambda: _bf16_dot(4, 600, 13651, 128)])
+def test_partial_sums_leave_room_for_the_other_temporaries(compile_client, program):
     # K ranges are taken as far as the partial sums fit the 64 MiB that an allocation-free execution has
-    exe, _ = _plan(compile_client, _swiglu(m, d, f))
+    exe, _ = _plan(compile_client, program())
     assert exe.executable().memory_statistics()["temp_size_in_bytes"] <= 64 << 20, exe.describe_plan()
 
 
