@@ -212,7 +212,7 @@ static bool edge_splittable(const GemmArgs& g, const Choice& c, int splits) {
 // CU to itself (`alone`) and per workgroup of a busy CU (`shared`), a workgroup's start and end (`round`), and storing 16384
 // bytes of its results (`store`). Fitted to the kernel times of 1950 products of drawn shapes (1 to 16000 rows, k 16 to 16000, up to
 // 16 at a time), every tile and number of K ranges of each, then adjusted where the choice was not the best one. Over those
-// shapes the choice takes 1.014 times the best one's time; 1.038 by the family's estimates below, which know neither the
+// shapes the choice takes 1.012 times the best one's time; 1.038 by the family's estimates below, which know neither the
 // results' bytes nor a workgroup's start (64×128 tiles stored the two results of 760 × 896 × 7936 i8 in 26 µs, 128×128 in
 // 21; f32 was split where it fills the chip, 16 × 3328 × 1264 × 48 132 µs, 103 unsplit). Small tiles move more operand bytes
 // per product (a 64×64 tile's k-tile takes 0.2 µs whether the CU runs one or eight of them: it is the L2-to-LDS rate, about
@@ -224,7 +224,7 @@ struct EdgeTime {
 };
 static constexpr EdgeTime kEdgeTimes[] = {
     {MMA_BF16, 256, 256, 0, 1.14, 1.28, 2.56, 0.29},     {MMA_BF16, 128, 128, 0, 0.85, 0.50, 1.49, 0.20},
-    {MMA_BF16, 64, 64, 0, 0.26, 0.23, 0.89, 0.00},       {MMA_BF16, 32, 128, 0, 0.06, 0.24, 1.31, 0.00},
+    {MMA_BF16, 64, 64, 0, 0.26, 0.23, 0.89, 0.00},       {MMA_BF16, 32, 128, 0, 0.30, 0.24, 1.31, 0.00},
     {MMA_F16, 128, 128, 0, 0.52, 0.44, 1.25, 0.47},      {MMA_F32, 64, 64, 0, 0.44, 0.36, 0.77, 0.12},
     {MMA_I8, 256, 256, 0, 1.16, 1.17, 3.81, 0.38},       {MMA_I8, 128, 128, 0, 0.70, 0.42, 1.94, 0.43},
     {MMA_I8, 64, 128, 0, 0.31, 0.40, 1.50, 0.51},        {MMA_I8, 32, 128, 0, 0.25, 0.24, 1.16, 0.26},
@@ -235,7 +235,7 @@ static constexpr EdgeTime kEdgeTimes[] = {
 
 // Estimated microseconds of an edge tile over `splits` K ranges: the busiest CU's workgroups, and for a split the reduction
 // launch, or (partial sums up to 8 MiB) the arrival and the finish, in which one workgroup sums and stores a tile by itself:
-// 5.5 µs for 128×128 elements, 17 with a scaled or SwiGLU epilogue.
+// 5 µs for 128×128 elements, 17 with a scaled or SwiGLU epilogue.
 static double edge_cost(const GemmArgs& g, int kind, const Choice& c, int splits) {
   const EdgeTime* t = nullptr;
   for (const EdgeTime& x : kEdgeTimes)
@@ -250,7 +250,7 @@ static double edge_cost(const GemmArgs& g, int kind, const Choice& c, int splits
   double us = 2.4 + per * std::max(t->alone, t->shared * busiest) + busiest * (t->round + t->store * stored);
   if (splits > 1) {
     const double mb = (double)gemm_partial_bytes(g, splits) / (1 << 20);
-    us += mb <= 8.0 ? 1.8 + 0.34 * mb + area * (g.epilogue == EPI_STORE ? 5.5 : 16.7) : 6.6 + 0.24 * mb;
+    us += mb <= 8.0 ? 2.0 + 0.34 * mb + area * (g.epilogue == EPI_STORE ? 5.0 : 16.7) : 6.6 + 0.24 * mb;
   }
   return us;
 }
