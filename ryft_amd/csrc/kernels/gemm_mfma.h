@@ -15,10 +15,10 @@
 //
 // Measured (kernel times, before: register-staged edge tiles of 128×128 only, loads issued behind a branch):
 // 1000³ bf16 17.3 → 8.4 µs (64×64 tiles), Xᵀ·dY of [2048, 4096]ᵀ·[2048, 4096] 103 → 59 µs (256×256, both operands by
-// transposing reads), 16 rows × f8 weights [4096, 14336] twice 77 → 30 µs and [14336, 4096] 172 → 18 µs (32×128 tiles
-// over K ranges). What bounds them: the 64×64 tiles the L2-to-LDS rate (about 60 GB/s per CU), the 32×128 tiles of f8 weights
-// the latency of their loads, a barrier per k-tile with too few bytes in flight (16 rows: gate and up 4.7 TB/s from HBM,
-// down 3.7, MFMA busy 12-16%, no LDS queue), the large ones the MFMA issue at the clock the chip holds.
+// transposing reads), 16 rows × f8 weights [4096, 14336] twice 77 → 26 µs and [14336, 4096] 172 → 18 µs (32×128 tiles
+// over K ranges). What bounds them: the 64×64 tiles the L2-to-LDS rate (about 70 GB/s per CU), the 32×128 tiles of f8 weights
+// the latency of their loads, a barrier per k-tile with too few bytes in flight (16 rows: gate and up 4.9 TB/s from HBM,
+// down 3.7, MFMA busy 12-17%, no LDS queue), the large ones the MFMA issue at the clock the chip holds.
 //
 // Instruction per compute type (all dense, f32 or i32 accumulation):
 //   bf16  v_mfma_f32_32x32x16_bf16      f16  v_mfma_f32_32x32x16_f16
